@@ -246,6 +246,10 @@ FusedModule::~FusedModule() {
     if (module) (void)hipModuleUnload(module);
 }
 
+RowsModule::~RowsModule() {
+    if (module) (void)hipModuleUnload(module);
+}
+
 ExpressionEpoch::~ExpressionEpoch() {
     if (module) (void)hipModuleUnload(module);
 }
@@ -266,6 +270,18 @@ static bool fused_eligible(const Net& n, const Plan& p) {
         if (n.linear[l] || n.neurons[l] > 256) return false;
     return n.neurons[L - 1] <= 8 && n.neurons[L - 1] <= n.neurons[L - 2];
 }
+
+static bool has_sigmoid(const Net& n) {
+    for (int l = 0; l + 1 < n.layers; ++l)
+        if (!n.linear[l]) return true;
+    return false;
+}
+
+// Rows up to which a plan outside the fused kernels composes in generated row
+// kernels instead of the table-driven ones.  At 126 rows (4 variables, order 5)
+// the adjoint takes 453 of a lane's 512 registers and the module compiles in
+// 5 s; at 210 (4 variables, order 6) it spills 334 of them and takes 44 s.
+constexpr int kRowsModuleRows = 128;
 
 static std::string device_arch(int ordinal) {
     hipDeviceProp_t prop;
@@ -435,6 +451,20 @@ static std::shared_ptr<FusedModule> load_fused(Device& d, const Tables& t, const
     return m;
 }
 
+static std::shared_ptr<RowsModule> load_rows(Device& d, const Tables& t) {
+    const std::string src = rows_source(t);
+    for (auto& kv : d.rows_modules)
+        if (kv.first == src) return kv.second;
+    std::string log;
+    const std::vector<char> code = compile_module(src, device_arch(d.ordinal), &log);
+    auto m = std::make_shared<RowsModule>();
+    HIP_CHECK(hipModuleLoadData(&m->module, code.data()));
+    HIP_CHECK(hipModuleGetFunction(&m->forward, m->module, "rows_forward_k"));
+    HIP_CHECK(hipModuleGetFunction(&m->adjoint, m->module, "rows_adjoint_k"));
+    d.rows_modules.emplace_back(src, m);
+    return m;
+}
+
 static void launch_module(Device& d, hipFunction_t f, unsigned gx, unsigned gy, void** args, unsigned threads = 256) {
     HIP_CHECK(hipModuleLaunchKernel(f, gx, gy, 1, threads, 1, 1, 0, d.stream, args, nullptr));
 }
@@ -454,6 +484,29 @@ static NetArgsHost net_args(const Plan& p) {
     a.X = p.input;
     a.Z[0] = p.input;
     return a;
+}
+
+// Compositions of a layer of n neurons outside the fused kernels: y from z, and
+// dE/dz from z and dE/dy in place.  The row kernels are straight-line code over
+// a lane's registers (the Taylor recurrence and correlation of the network
+// kernels on unscaled stacks), bound by the stacks' bytes; the table-driven
+// kernels walk every partition of every row from memory.  3->64^3->1 at order 6
+// (84 rows) over 2,000 points, a layer's adjoint 833 -> 39 us (3.3 TB/s at one
+// wave per SIMD) and forward 381 -> under 20 us, the epoch 4,226 -> 731 us;
+// 2->512^3->1 at order 2, 2,048-point chunks, 26 -> 12 and 17 -> 9 us.
+static void compose_forward(Device& d, const Plan& p, const float* z, float* y, int n) {
+    if (!p.rows_module) return launch_compose_forward(d, p, z, y, n);
+    int elements = p.width * n;
+    TraceScope trace(d, kTraceComposeForward, 8.0 * double(elements) * p.rows);
+    void* args[] = {&z, &y, &n, &elements};
+    launch_module(d, p.rows_module->forward, unsigned((elements + 255) / 256), 1, args);
+}
+static void compose_adjoint(Device& d, const Plan& p, const float* z, float* g, int n) {
+    if (!p.rows_module) return launch_compose_adjoint(d, p, z, g, n);
+    int elements = p.width * n;
+    TraceScope trace(d, kTraceComposeAdjoint, 12.0 * double(elements) * p.rows);
+    void* args[] = {&z, &g, &n, &elements};
+    launch_module(d, p.rows_module->adjoint, unsigned((elements + 255) / 256), 1, args);
 }
 
 struct GradientPlan;
@@ -1416,6 +1469,8 @@ int cpde_plan_create(cpde_net* net, int rows, int variables, const int* table, i
         if (fused_eligible(*net, *p)) {
             p->fused = load_fused(*net->dev, p->tables, net->neurons, width);
             p->network = network_mode();
+        } else if (p->rows <= kRowsModuleRows && env_int("CPDE_FUSED", 1) && has_sigmoid(*net)) {
+            p->rows_module = load_rows(*net->dev, p->tables);
         }
         sync_stream(*net->dev, __LINE__);
         *out = p.release();
@@ -1561,7 +1616,7 @@ int cpde_forward(cpde_plan* plan) {
         const int cols = int(plan->columns());
         for (int t = 0; t + 1 < n.layers; ++t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
-            if (!n.linear[t]) launch_compose_forward(d, *plan, n.z[t], n.y[t], ni);
+            if (!n.linear[t]) compose_forward(d, *plan, n.z[t], n.y[t], ni);
             const float* W = n.state[0][t];
             launch_gemm(d, no, cols, ni, W, no, false, activations(*plan, t), ni, false, n.z[t + 1], no,
                         W + size_t(no) * ni, plan->rows);
@@ -1725,7 +1780,7 @@ int cpde_backward(cpde_plan* plan, int accumulate) {
         for (int t = n.layers - 2; t >= 1; --t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
             launch_gemm(d, ni, cols, no, n.state[0][t], no, true, n.g[t + 1], no, false, n.g[t], ni, nullptr, 1);
-            if (!n.linear[t]) launch_compose_adjoint(d, *plan, n.z[t], n.g[t], ni);
+            if (!n.linear[t]) compose_adjoint(d, *plan, n.z[t], n.g[t], ni);
         }
         weight_gradients(*plan, accumulate != 0);
     });

@@ -93,6 +93,7 @@ Tables build_tables(int rows, int variables, const int* table);
 
 struct Device;
 struct FusedModule;
+struct RowsModule;
 struct ExpressionEpoch;
 
 struct Net {
@@ -145,7 +146,8 @@ struct Plan {
     // the plan's activated chunk [point][row][channel] (layer 0): its own, so
     // that plans of one network keep their inputs between epochs
     float* input = nullptr;
-    std::shared_ptr<FusedModule> fused;  // null: table-driven kernels
+    std::shared_ptr<FusedModule> fused;  // null: one launch per product and composition
+    std::shared_ptr<RowsModule> rows_module;  // their compositions (null: table-driven)
     bool network = false;                // fused: one network-wide kernel per pass
     CostStats* epoch_partials = nullptr;  // one-pass epoch: one cost record per workgroup, two sets
     int epoch_capacity = 0, epoch_turn = 0;
@@ -293,6 +295,7 @@ struct Device {
     void fold_trace();
     // fused modules compiled on this device, by source text
     std::vector<std::pair<std::string, std::shared_ptr<FusedModule>>> fused_modules;
+    std::vector<std::pair<std::string, std::shared_ptr<RowsModule>>> rows_modules;
     std::vector<std::pair<std::string, std::shared_ptr<ExpressionEpoch>>> expression_epochs;
     // Cost slots cleared by cpde_costs_begin and not yet written: the first
     // finish into a slot overwrites it instead of accumulating.
@@ -367,6 +370,14 @@ struct FusedModule {
     ~FusedModule();
 };
 std::string compose_source(const Tables& t, const std::vector<int>& splits, bool scaled = false);
+// Compositions of one schema over whole stacks (rows_source): y from z, and
+// dE/dz from z and dE/dy in place.
+struct RowsModule {
+    hipModule_t module = nullptr;
+    hipFunction_t forward = nullptr, adjoint = nullptr;
+    ~RowsModule();
+};
+std::string rows_source(const Tables& t);
 // Launch-shape choices of the fused kernels (environment overrides in api.hip).
 struct FusedTuning {
     int points_per_block = 2;      // layer-fused kernels

@@ -302,9 +302,14 @@ struct Jet {
 
 // y[0] = sigma(z0), u[0] = sigma'(z0) = sigma(z0) sigma(-z0) and c0 = 1 - 2 sigma(z0)
 // from e^{-|z0|}, which cannot overflow; no cancellation at either tail.
-void emit_scaled_sigmoid(std::ostringstream& o) {
-    o << "    const float E = __expf(-fabsf(z[0]));\n"
-         "    const float sp = __builtin_amdgcn_rcpf(1.0f + E);\n"  // sigma(|z0|)
+// `rounded`: the library's exponential and a true division instead of the
+// hardware's approximations (for the row kernels, which wait on memory).
+void emit_scaled_sigmoid(std::ostringstream& o, bool rounded) {
+    o << (rounded ? "    const float E = expf(-fabsf(z[0]));\n"
+                    "    const float sp = 1.0f / (1.0f + E);\n"
+                  : "    const float E = __expf(-fabsf(z[0]));\n"
+                    "    const float sp = __builtin_amdgcn_rcpf(1.0f + E);\n")  // sigma(|z0|)
+      <<
          "    const float sn = E * sp;\n"                           // sigma(-|z0|)
          "    const bool pos = z[0] >= 0.0f;\n"
          "    y[0] = pos ? sp : sn;\n"
@@ -317,11 +322,12 @@ void emit_scaled_sigmoid(std::ostringstream& o) {
 // takes the others from its partner lane (the adjacent lane, which runs the
 // same code on the jet with variables 0 and 1 swapped, so its row mirror(b)
 // is this lane's row b).
-void emit_scaled_forward(std::ostringstream& o, const Tables& t, const std::string& name, bool mirror) {
+void emit_scaled_forward(std::ostringstream& o, const Tables& t, const std::string& name, bool mirror,
+                         bool rounded = false) {
     const Jet J(t);
     o << "__device__ __forceinline__ void " << name
       << "(const float* __restrict__ z, float* __restrict__ y, float* __restrict__ u) {\n";
-    emit_scaled_sigmoid(o);
+    emit_scaled_sigmoid(o, rounded);
     std::map<std::pair<int, int>, std::string> directional;  // (i, r) -> delta_i * z[r]
     auto zdir = [&](int i, int r) -> std::string {
         const int d = J.alpha[r][i];
@@ -406,6 +412,15 @@ void emit_scaled_adjoint(std::ostringstream& o, const Tables& t, const std::stri
     o << "}\n";
 }
 
+// alpha! of every row.
+std::vector<float> row_factorials(const Jet& J) {
+    std::vector<float> fact(J.R, 1.0f);
+    for (int r = 0; r < J.R; ++r)
+        for (int c : J.alpha[r])
+            for (int k = 2; k <= c; ++k) fact[r] *= float(k);
+    return fact;
+}
+
 int scaled_adjoint_terms(const Jet& J, int b) {
     int n = 1;
     for (int a = b + 1; a < J.R; ++a) n += Jet::below(J.alpha[b], J.alpha[a]);
@@ -439,10 +454,7 @@ std::string compose_source(const Tables& t, const std::vector<int>& splits, bool
     emit_adjoint(o, t, "compose_adjoint", all);
     if (scaled) {
         const Jet J(t);
-        std::vector<float> fact(t.rows, 1.0f);
-        for (int r = 0; r < t.rows; ++r)
-            for (int c : J.alpha[r])
-                for (int k = 2; k <= c; ++k) fact[r] *= float(k);
+        const std::vector<float> fact = row_factorials(J);
         o << "constexpr float kRowScale[" << t.rows << "] = {";
         for (int r = 0; r < t.rows; ++r) o << (r ? ", " : "") << flit(fact[r]);
         o << "};\n__constant__ float kRowScaleTable[" << t.rows << "] = {";
@@ -503,6 +515,61 @@ std::string compose_source(const Tables& t, const std::vector<int>& splits, bool
             }
         }
     }
+    return o.str();
+}
+
+// Compositions of a schema as kernels over whole stacks, for the plans that the
+// fused kernels do not take: one lane per (point, neuron), its rows in
+// registers, unscaled stacks on both sides.  rows_forward_k: y from z.
+// rows_adjoint_k: dE/dz from z and dE/dy, in place over the latter; the jet of
+// sigma'(z) is formed again from z, and the adjoint's loads follow it so that
+// z, y and u need not stay live beside dE/dy.
+std::string rows_source(const Tables& t) {
+    const Jet J(t);
+    const std::vector<float> fact = row_factorials(J);
+    std::ostringstream o;
+    o << "// generated: compositions over stacks\n#define R " << t.rows << "\n";
+    auto table = [&](const char* name, bool inverse) {
+        o << "constexpr float " << name << "[R] = {";
+        for (int r = 0; r < t.rows; ++r) o << (r ? ", " : "") << flit(inverse ? 1.0f / fact[r] : fact[r]);
+        o << "};\n";
+    };
+    table("kScale", false);
+    table("kUnscale", true);
+    emit_scaled_forward(o, t, "compose", false, true);
+    emit_scaled_adjoint(o, t, "adjoint", std::vector<char>(t.rows, 1));
+    o << R"(
+extern "C" __global__ __launch_bounds__(256) void rows_forward_k(const float* __restrict__ Z, float* __restrict__ Y,
+                                                                 int n, int elements) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= elements) return;
+    const int p = e / n;
+    const size_t base = size_t(p) * R * n + (e - p * n);
+    float z[R], y[R], u[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) z[r] = Z[base + size_t(r) * n] * kUnscale[r];
+    compose(z, y, u);
+#pragma unroll
+    for (int r = 0; r < R; ++r) Y[base + size_t(r) * n] = y[r] * kScale[r];
+}
+extern "C" __global__ __launch_bounds__(256) void rows_adjoint_k(const float* __restrict__ Z, float* __restrict__ G,
+                                                                 int n, int elements) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= elements) return;
+    const int p = e / n;
+    const size_t base = size_t(p) * R * n + (e - p * n);
+    float z[R], y[R], u[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) z[r] = Z[base + size_t(r) * n] * kUnscale[r];
+    compose(z, y, u);
+    float gy[R], gz[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) gy[r] = G[base + size_t(r) * n] * kScale[r];
+    adjoint(u, gy, gz);
+#pragma unroll
+    for (int r = 0; r < R; ++r) G[base + size_t(r) * n] = gz[r] * kUnscale[r];
+}
+)";
     return o.str();
 }
 
