@@ -486,6 +486,11 @@ static NetArgsHost net_args(const Plan& p) {
     return a;
 }
 
+// Outputs up to which a transition outside the fused kernels takes a wave per
+// column and dot product instead of a matrix tile of 64 rows (512 -> 1 over
+// 12,288 columns: 76 us as a tile of the fp32 product, 8.8 us).
+constexpr int kOutputForwardMax = 8;
+
 // Compositions of a layer of n neurons outside the fused kernels: y from z, and
 // dE/dz from z and dE/dy in place.  The row kernels are straight-line code over
 // a lane's registers (the Taylor recurrence and correlation of the network
@@ -1618,8 +1623,11 @@ int cpde_forward(cpde_plan* plan) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
             if (!n.linear[t]) compose_forward(d, *plan, n.z[t], n.y[t], ni);
             const float* W = n.state[0][t];
-            launch_gemm(d, no, cols, ni, W, no, false, activations(*plan, t), ni, false, n.z[t + 1], no,
-                        W + size_t(no) * ni, plan->rows);
+            if (no <= kOutputForwardMax)
+                launch_output_forward(d, W, activations(*plan, t), n.z[t + 1], ni, no, plan->rows, cols);
+            else
+                launch_gemm(d, no, cols, ni, W, no, false, activations(*plan, t), ni, n.z[t + 1], no,
+                            W + size_t(no) * ni, plan->rows);
         }
     });
 }
@@ -1779,7 +1787,7 @@ int cpde_backward(cpde_plan* plan, int accumulate) {
         const int cols = int(plan->columns());
         for (int t = n.layers - 2; t >= 1; --t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
-            launch_gemm(d, ni, cols, no, n.state[0][t], no, true, n.g[t + 1], no, false, n.g[t], ni, nullptr, 1);
+            launch_gemm(d, ni, cols, no, n.state[0][t], no, true, n.g[t + 1], no, n.g[t], ni, nullptr, 1);
             if (!n.linear[t]) compose_adjoint(d, *plan, n.z[t], n.g[t], ni);
         }
         weight_gradients(*plan, accumulate != 0);

@@ -426,11 +426,11 @@ void launch_output(Device& d, float* dest, const float* out, int dest_width, int
                    int rows, int width, int offset, int valid);
 void launch_compose_forward(Device& d, const Plan& p, const float* z, float* y, int n);
 void launch_compose_adjoint(Device& d, const Plan& p, const float* z, float* g, int n);
-// C[M x N] = A[M x K] * B[K x N]; a_t: A stored k-contiguous (A[k + lda*m]);
-// b_t: B stored n-contiguous (B[n + ldb*k]).  bias (may be null) is added to every
-// column n with n % period == 0.
-void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_t, const float* B, int ldb, bool b_t,
-                 float* C, int ldc, const float* bias, int period);
+// C[M x N] = A[M x K] B[N x K]^T: B k-contiguous (B[k + ldb*n]), A k-contiguous
+// (a_k: A[k + lda*m]) or m-contiguous (A[m + lda*k]), C[m + ldc*n].  bias (may be
+// null) is added to every column n with n % period == 0.
+void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_k, const float* B, int ldb, float* C,
+                 int ldc, const float* bias, int period);
 void launch_matching(Device& d, const Plan& p, const float* y, float* g, const float* target, int target_width,
                      const int* target_rows, const float* weights, int weight_samples, int offset, int valid,
                      int cost_index, bool collect, bool gradient);

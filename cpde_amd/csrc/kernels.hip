@@ -169,117 +169,6 @@ void launch_compose_adjoint(Device& d, const Plan& p, const float* z, float* g, 
 }
 
 // ------------------------------------------------------------------------------------------
-// FP32 MFMA GEMM: C[M x N] = A[M x K] * B[K x N] on v_mfma_f32_32x32x2_f32 (true
-// fp32, no reduced-precision shortcut).  256 lanes = WM x WN waves; each wave owns
-// a (BM/WM) x (BN/WN) tile made of 32x32 MFMA blocks.  Tiles of A and B pass
-// through LDS in K chunks of BK.  Split-K: blockIdx.z takes K range
-// [z*k_split, (z+1)*k_split) and writes its partial product to C + z*ldc*N.
-constexpr int BK = 16;
-
-template <int BM, int BN, int WM, int WN>
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda, int a_t,
-                                                   const float* __restrict__ Bm, int ldb, int b_t, float* __restrict__ C,
-                                                   int ldc, const float* __restrict__ bias, int period, int k_split) {
-    constexpr int TM = BM / WM, TN = BN / WN;
-    constexpr int IM = TM / 32, IN = TN / 32;
-    __shared__ float As[BK][BM + 1];
-    __shared__ float Bs[BK][BN + 1];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = wave % WM, wn = wave / WM;
-    const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-    int kbegin = 0, kend = K;
-    if (k_split > 0) {
-        kbegin = blockIdx.z * k_split;
-        kend = min(K, kbegin + k_split);
-        C += size_t(blockIdx.z) * ldc * N;
-    }
-    floatx16 acc[IM][IN];
-#pragma unroll
-    for (int a = 0; a < IM; ++a)
-#pragma unroll
-        for (int b = 0; b < IN; ++b)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
-
-    for (int k0 = kbegin; k0 < kend; k0 += BK) {
-        // A tile -> As[k][m]
-#pragma unroll
-        for (int idx = t; idx < BM * BK; idx += 256) {
-            int m, k;
-            if (a_t) { k = idx % BK; m = idx / BK; }
-            else { m = idx % BM; k = idx / BM; }
-            const int gm = m0 + m, gk = k0 + k;
-            float v = 0.0f;
-            if (gm < M && gk < kend) v = a_t ? A[gk + size_t(lda) * gm] : A[gm + size_t(lda) * gk];
-            As[k][m] = v;
-        }
-        // B tile -> Bs[k][n]
-#pragma unroll
-        for (int idx = t; idx < BN * BK; idx += 256) {
-            int n, k;
-            if (b_t) { n = idx % BN; k = idx / BN; }
-            else { k = idx % BK; n = idx / BK; }
-            const int gn = n0 + n, gk = k0 + k;
-            float v = 0.0f;
-            if (gn < N && gk < kend) v = b_t ? Bm[gn + size_t(ldb) * gk] : Bm[gk + size_t(ldb) * gn];
-            Bs[k][n] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            const int kr = kk + (lane >> 5), lc = lane & 31;
-            float av[IM], bv[IN];
-#pragma unroll
-            for (int a = 0; a < IM; ++a) av[a] = As[kr][wm * TM + a * 32 + lc];
-#pragma unroll
-            for (int b = 0; b < IN; ++b) bv[b] = Bs[kr][wn * TN + b * 32 + lc];
-#pragma unroll
-            for (int a = 0; a < IM; ++a)
-#pragma unroll
-                for (int b = 0; b < IN; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a], bv[b], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // Accumulator layout of a 32x32 block: lane l, register v holds
-    // row 8*(v/4) + 4*(l/32) + v%4, column l%32.
-#pragma unroll
-    for (int a = 0; a < IM; ++a)
-#pragma unroll
-        for (int b = 0; b < IN; ++b) {
-            const int gn = n0 + wn * TN + b * 32 + (lane & 31);
-            if (gn >= N) continue;
-            const bool add_bias = bias != nullptr && (gn % period) == 0;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int gm = m0 + wm * TM + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (gm < M) C[gm + size_t(ldc) * gn] = acc[a][b][v] + (add_bias ? bias[gm] : 0.0f);
-            }
-        }
-}
-
-static void gemm_dispatch(Device& d, int M, int N, int K, const float* A, int lda, bool a_t, const float* B, int ldb,
-                          bool b_t, float* C, int ldc, const float* bias, int period, int splits, int k_split) {
-    if (M <= 32) {
-        dim3 grid((M + 31) / 32, (N + 127) / 128, splits);
-        hipLaunchKernelGGL((gemm_kernel<32, 128, 1, 4>), grid, 256, 0, d.stream, M, N, K, A, lda, int(a_t), B, ldb,
-                           int(b_t), C, ldc, bias, period, k_split);
-    } else {
-        dim3 grid((M + 127) / 128, (N + 63) / 64, splits);
-        hipLaunchKernelGGL((gemm_kernel<128, 64, 4, 1>), grid, 256, 0, d.stream, M, N, K, A, lda, int(a_t), B, ldb,
-                           int(b_t), C, ldc, bias, period, k_split);
-    }
-    HIP_CHECK(hipGetLastError());
-}
-
-void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_t, const float* B, int ldb, bool b_t,
-                 float* C, int ldc, const float* bias, int period) {
-    if (M <= 0 || N <= 0) return;
-    TraceScope trace(d, a_t ? kTraceGemmTransposed : kTraceGemm, 2.0 * M * double(N) * K);
-    gemm_dispatch(d, M, N, K, A, lda, a_t, B, ldb, b_t, C, ldc, bias, period > 0 ? period : 1, 1, 0);
-}
-
-// ------------------------------------------------------------------------------------------
 // Output transition with few outputs: z[col][o] = sum_i W[o + NO*i] y[col][i]
 // (+ bias on value-row columns).  One wave per column, lanes stride the inputs,
 // fixed-order wave reduction.
@@ -526,6 +415,249 @@ __device__ __forceinline__ int group_of(const int (&begin)[kMaxTransitions + 1],
 __device__ __forceinline__ int xcd_grouped(int b, int n) {
     const int x = b & 7, q = b >> 3, per = (n + 7) >> 3, full = (n & 7) ? (n & 7) : 8;
     return x < full ? x * per + q : full * per + (x - full) * (per - 1) + q;
+}
+
+// ------------------------------------------------------------------------------------------
+// Matrix products of fp32 operands on the bf16 matrix cores, at fp32 accuracy.
+// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 significant
+// bits): x = x1 + x2 + x3, x1 its upper half, x2 the rest rounded to nearest,
+// x3 what remains.  Of the nine products of two such sums, six matter at 24
+// bits: x1 y1 goes into one accumulator and x1 y2 + x2 y1 + x2 y2 + x1 y3 +
+// x3 y1 into another, so that the small terms are not rounded to the large
+// sum's last place; the two meet once at the end.  v_mfma_f32_16x16x32_bf16
+// runs at 2,100 TFLOP/s here and v_mfma_f32_16x16x4_f32 at 153, so six of
+// them cost 0.44 of one fp32 product, and bf16 products overlap with other
+// waves' vector instructions, which fp32 ones do not (0.26 + 0.91 ms alone,
+// 1.00 together; fp32 0.22 + 0.91, 1.13).  Relative error of a product
+// against 64 bits: 128 random terms 6.0e-8 (fp32 instruction 1.9e-7), 28,672
+// terms of one sign 8.6e-7 (2.4e-6; 7.1e-6 with one accumulator for all six).
+// An infinite operand gives NaN where fp32 gave an infinity (inf - inf).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+// The upper halves of two words, the first in the lower half.
+__device__ __forceinline__ unsigned upper_halves(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ __forceinline__ float upper_half(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+
+// Eight values into their three planes.
+__device__ __forceinline__ void split_planes(const float (&x)[8], uintx4 (&plane)[3]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = x[2 * i], b = x[2 * i + 1];
+        const float ra = a - upper_half(a), rb = b - upper_half(b);
+        const bf16x2 mid = __builtin_convertvector(floatx2{ra, rb}, bf16x2);
+        const unsigned m = __builtin_bit_cast(unsigned, mid);
+        plane[0][i] = upper_halves(a, b);
+        plane[1][i] = m;
+        plane[2][i] = upper_halves(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+    }
+}
+
+// One 64 WM x 64 WN tile of A B^T over k in [kbegin, kend): four waves, each a
+// 64 x 64 block of sixteen 16 x 16 products.  An operand's rows pass through LDS
+// in steps of 32 columns of k, split on the way in, laid out as the matrix
+// instruction reads them: for 16 rows, three planes of 64 lanes x 16 bytes
+// (lane (q, j): row j, k = 8q .. 8q + 7), so the reads are contiguous; 16 rows
+// take 16 bytes more, which spreads the transposing writes over the banks.
+// K_MAJOR: operand element (row, k) at p[k + ld * row], a thread takes eight
+// consecutive k of a row; otherwise at p[row + ld * k], a thread takes one or
+// two adjacent rows of eight k's, so that a wave reads whole lines of each k.
+// VEC: float4 and float2 loads (ld and the operand's extents multiples of 4,
+// the base aligned to 16 bytes).  Rows beyond `rows` and
+// k beyond kend are zero.
+constexpr int kSpRows16 = 3 * 1024 + 16;  // bytes of 16 rows of one 32-column step
+constexpr int sp_lds_bytes(int rows) { return rows / 16 * kSpRows16; }
+
+// A thread's share of ROWS x 32 elements among the workgroup's 256 threads:
+// chunks of eight k's, of rows 16 apart (K_MAJOR) or adjacent (not).
+template <int ROWS, bool K_MAJOR, bool VEC>
+struct SplitStage {
+    static constexpr int kChunks = ROWS / 64;
+    static_assert(ROWS % 64 == 0 && (K_MAJOR || kChunks <= 2), "whole chunks per thread");
+    float raw[kChunks][8];
+
+    __device__ __forceinline__ void load(const float* __restrict__ p, int ld, int rows, int row0, int k0, int kend,
+                                         int tid) {
+        if constexpr (K_MAJOR) {
+#pragma unroll
+            for (int c = 0; c < kChunks; ++c) {
+                const int s = tid + 256 * c, row = row0 + (s >> 6) * 16 + (s & 15), k = k0 + 8 * ((s >> 4) & 3);
+                const float* src = p + size_t(ld) * row + k;
+                if constexpr (VEC) {
+                    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const floatx4 lo = row < rows && k < kend ? *reinterpret_cast<const floatx4*>(src) : zero;
+                    const floatx4 hi = row < rows && k + 4 < kend ? *reinterpret_cast<const floatx4*>(src + 4) : zero;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        raw[c][i] = lo[i];
+                        raw[c][4 + i] = hi[i];
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) raw[c][i] = row < rows && k + i < kend ? src[i] : 0.0f;
+                }
+            }
+        } else {
+            const int row = row0 + kChunks * (tid & 63), k = k0 + 8 * (tid >> 6);
+            const float* src = p + row + size_t(ld) * k;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if constexpr (kChunks == 2 && VEC) {
+                    floatx2 v = {0.0f, 0.0f};
+                    if (k + i < kend && row < rows) v = *reinterpret_cast<const floatx2*>(src + size_t(ld) * i);
+                    raw[0][i] = v[0];
+                    raw[1][i] = v[1];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < kChunks; ++r)
+                        raw[r][i] = k + i < kend && row + r < rows ? src[size_t(ld) * i + r] : 0.0f;
+                }
+            }
+        }
+    }
+
+    __device__ __forceinline__ void store(unsigned char* lds, int tid) const {
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+            const int s = tid + 256 * c;
+            const int row = K_MAJOR ? (s >> 6) * 16 + (s & 15) : kChunks * (tid & 63) + c;
+            const int q = K_MAJOR ? (s >> 4) & 3 : tid >> 6;
+            uintx4 plane[3];
+            split_planes(raw[c], plane);
+            unsigned char* dst = lds + (row >> 4) * kSpRows16 + q * 256 + (row & 15) * 16;
+#pragma unroll
+            for (int x = 0; x < 3; ++x) *reinterpret_cast<uintx4*>(dst + 1024 * x) = plane[x];
+        }
+    }
+};
+
+// The accumulators of a wave's 64 x 64 block: big + small is the product;
+// register v of lane (q, j) of (a, b) is row 16a + 4q + v, column 16b + j.
+struct SplitBlock {
+    floatx4 big[4][4], small[4][4];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) big[a][b] = small[a][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+};
+
+// One step's products from the staged rows (A: 4 x 16 rows at la, B at lb).
+__device__ __forceinline__ void split_products(SplitBlock& c, const unsigned char* la, const unsigned char* lb,
+                                               int lane) {
+    bf16x8 a[4][3];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+            a[x][s] = *reinterpret_cast<const bf16x8*>(la + x * kSpRows16 + 1024 * s + 16 * lane);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+        bf16x8 b[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) b[s] = *reinterpret_cast<const bf16x8*>(lb + y * kSpRows16 + 1024 * s + 16 * lane);
+        // four independent accumulators between dependent products
+#define CPDE_SPLIT_TERM(acc, i, k) \
+    _Pragma("unroll") for (int x = 0; x < 4; ++x) \
+        c.acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x][i], b[k], c.acc[x][y], 0, 0, 0);
+        CPDE_SPLIT_TERM(small, 0, 2)
+        CPDE_SPLIT_TERM(big, 0, 0)
+        CPDE_SPLIT_TERM(small, 2, 0)
+        CPDE_SPLIT_TERM(small, 1, 1)
+        CPDE_SPLIT_TERM(small, 0, 1)
+        CPDE_SPLIT_TERM(small, 1, 0)
+#undef CPDE_SPLIT_TERM
+    }
+}
+
+// C[M x N] = A[M x K] B[N x K]^T, B k-contiguous, A k-contiguous (A_K) or
+// m-contiguous, C m-contiguous, with `bias` added to every column n with n %
+// period == 0.  Tiles of 128 x 128, or 64 x 256 for M up to 64; two workgroups
+// per CU, so that one's loads, conversions and barriers run under the other's
+// products, the next step's loads in flight during a step's products.  512 x
+// 512 over 12,288 columns: 52 us, against 114 us of the fp32 instruction
+// (32 x 32 x 2, 16-column steps, scalar LDS traffic); 64 x 64 over 168,000
+// columns (M up to 64) 62 -> 22 to 29 us.
+template <bool A_K, bool VEC, int WM>
+__global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
+                                                            const float* __restrict__ B, int ldb, float* __restrict__ C,
+                                                            int ldc, const float* __restrict__ bias, int period) {
+    constexpr int WN = 4 / WM, TM = 64 * WM, TN = 64 * WN;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[sp_lds_bytes(TM + TN)];
+    unsigned char* const la = lds;
+    unsigned char* const lb = lds + sp_lds_bytes(TM);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tiles_m = (M + TM - 1) / TM;
+    const int block = xcd_grouped(int(blockIdx.x), int(gridDim.x));  // the tiles of the same B rows on one XCD
+    const int m0 = (block % tiles_m) * TM, n0 = (block / tiles_m) * TN;
+    SplitStage<TM, A_K, VEC> sa;
+    SplitStage<TN, true, VEC> sb;
+    auto load = [&](int k0) {
+        sa.load(A, lda, M, m0, k0, K, tid);
+        sb.load(B, ldb, N, n0, k0, K, tid);
+    };
+    SplitBlock c;
+    c.clear();
+    load(0);
+    for (int k0 = 0; k0 < K; k0 += 32) {
+        sa.store(la, tid);
+        sb.store(lb, tid);
+        __syncthreads();
+        if (k0 + 32 < K) load(k0 + 32);
+        split_products(c, la + (wave % WM) * sp_lds_bytes(64), lb + (wave / WM) * sp_lds_bytes(64), lane);
+        __syncthreads();
+    }
+    const int q = lane >> 4, j = lane & 15;
+    const int mw = m0 + 64 * (wave % WM) + 4 * q, nw = n0 + 64 * (wave / WM) + j;
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+        const int n = nw + 16 * y;
+        if (n >= N) break;
+        const bool add = bias != nullptr && n % period == 0;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int m = mw + 16 * x;
+            floatx4 v = c.big[x][y] + c.small[x][y];
+            float* dst = C + m + size_t(ldc) * n;
+            if (VEC && m + 4 <= M) {  // ldc is a multiple of 4 with the A operand's extent
+                if (add) v += *reinterpret_cast<const floatx4*>(bias + m);
+                *reinterpret_cast<floatx4*>(dst) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (m + r < M) dst[r] = v[r] + (add ? bias[m + r] : 0.0f);
+            }
+        }
+    }
+}
+
+template <bool A_K, bool VEC>
+static void split_gemm(Device& d, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+                       int ldc, const float* bias, int period) {
+    if (M <= 64)
+        hipLaunchKernelGGL((split_gemm_kernel<A_K, VEC, 1>), (N + 255) / 256, 256, 0, d.stream, M, N, K, A, lda, B, ldb,
+                           C, ldc, bias, period);
+    else
+        hipLaunchKernelGGL((split_gemm_kernel<A_K, VEC, 2>), (M + 127) / 128 * ((N + 127) / 128), 256, 0, d.stream, M,
+                           N, K, A, lda, B, ldb, C, ldc, bias, period);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_k, const float* B, int ldb, float* C,
+                 int ldc, const float* bias, int period) {
+    if (M <= 0 || N <= 0) return;
+    TraceScope trace(d, a_k ? kTraceGemmTransposed : kTraceGemm, 2.0 * M * double(N) * K);
+    const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    const bool vec = M % 4 == 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A) &&
+                     aligned(B) && aligned(C) && aligned(bias);
+    const auto run = a_k ? (vec ? split_gemm<true, true> : split_gemm<true, false>)
+                         : (vec ? split_gemm<false, true> : split_gemm<false, false>);
+    run(d, M, N, K, A, lda, B, ldb, C, ldc, bias, period > 0 ? period : 1);
 }
 
 // Two workgroups per CU (LDS 2 x 67.6 KB): one's chunk loads and barriers
