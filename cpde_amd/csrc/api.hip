@@ -602,6 +602,17 @@ static int wgrad_blocks_per_cu() { return std::max(1, env_int("CPDE_WGRAD_OCC", 
 // 0.0936/0.0954, 0.1033/0.1050; the Poisson graph epoch 0.0924 against 0.0943.
 static int wgrad_direct_blocks_per_cu() { return std::max(1, env_int("CPDE_WGRAD_DIRECT_OCC", 1)); }
 
+static int epoch_blocks(const Plan& p);
+static bool one_pass_fits(const Plan& p);
+
+// Bytes of a one-pass epoch's cost records at the front of the static scratch,
+// and the floats left behind them for split partials.
+static size_t static_record_bytes(int blocks) { return (sizeof(CostStats) * size_t(blocks) + 255) / 256 * 256; }
+static size_t static_partial_floats(int blocks) {
+    const size_t records = static_record_bytes(blocks);
+    return records < size_t(CPDE_STATIC_SCRATCH_BYTES) ? (size_t(CPDE_STATIC_SCRATCH_BYTES) - records) / sizeof(float) : 0;
+}
+
 // The gradient plan of transitions [first, first + count), count at most
 // kMaxTransitions (one grouped launch and one reduction); external_splits is
 // indexed by the absolute transition.
@@ -621,8 +632,10 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     // 128x128 splits would be short (fewer than kWgradMinColumns columns each):
     // then four times the tiles give each split four times the columns, and
     // the split partials the reduction reads shrink fourfold
-    bool small_tiles = false, direct = false;
+    bool small_tiles = false, direct = false, split = false, has256 = false;
+    auto wide = [&](int k) { return n.neurons[first + k + 1] > 64 && n.neurons[first + k] > 64; };
     auto tile_of = [&](int k) {
+        if (split && wide(k)) return std::max(n.neurons[first + k + 1], n.neurons[first + k]) > 128 ? 256 : 128;
         return direct || small_tiles || (n.neurons[first + k + 1] <= 64 && n.neurons[first + k] <= 64) ? 64 : 128;
     };
     auto tiles_of = [&](int k) {
@@ -637,7 +650,9 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     };
     // whole waves of tiles: a partial last wave would run alone for a whole split
     auto splits_for = [&](int tiles) {
-        const int per_cu = direct ? wgrad_direct_blocks_per_cu() : wgrad_blocks_per_cu();
+        int per_cu = direct ? wgrad_direct_blocks_per_cu() : wgrad_blocks_per_cu();
+        // two split tiles of 128 share a CU where that leaves them long
+        if (split && !has256 && double(K) * tiles >= 2.0 * 2048 * d.compute_units) per_cu = 2;
         return std::max(1, per_cu * d.compute_units / std::max(1, tiles));
     };
     int total_tiles = count_tiles();
@@ -650,13 +665,53 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     if (total_tiles > 0 && !staged) {
         small_tiles = true;
         direct = true;
+        // Split tiles (bf16 matrix instructions at fp32 accuracy) for transitions
+        // wider than 64 on both sides: 256x256 where a side is wider than 128,
+        // else 128x128 where a tile's split stays long.  2->256^4->1 over 65,536-point
+        // chunks 24.9 -> 15.8 ms of weight gradient per epoch (19.1 with 128x128
+        // tiles, two per CU); 3->128^5->1 over 32,768 points 1.32 -> 0.98 ms, the
+        // stacks' bytes at the rate of a copy; 2->512^3->1 over 12,288 columns 525 ->
+        // 98 us.  With 240 columns a split (2->128^4->1, 20,412 columns) the direct
+        // tiles stay ahead, 22 against 27 us: a split tile then writes four times the
+        // partials, and the reduction grows from 5 to 9 us.  CPDE_WGRAD_SPLIT=0 keeps the
+        // direct tiles everywhere.
+        for (int k = 0; k < T; ++k) {
+            const int M = n.neurons[first + k + 1], N = n.neurons[first + k];
+            if (external_splits[first + k] || !wide(k)) continue;
+            split = true;
+            has256 = has256 || std::max(M, N) > 128;
+        }
+        if (split) total_tiles = count_tiles();
+        if (split && !has256 && double(K) * total_tiles < 512.0 * d.compute_units) split = false;
+        if (!env_int("CPDE_WGRAD_SPLIT", 1)) split = false;
         total_tiles = count_tiles();
     } else if (total_tiles > 0 && K / splits_for(total_tiles) < kWgradMinColumns) {
         small_tiles = true;
         total_tiles = count_tiles();
     }
-    g.wa.direct = direct ? 1 : 0;
-    const int tile_splits = splits_for(total_tiles);
+    // transition k's splits, each of *chunk columns
+    auto splits_of = [&](int k, int* chunk) {
+        int s = external_splits[first + k];
+        if (s) return s;
+        s = thin(k) ? 2 * d.compute_units : splits_for(total_tiles);
+        s = std::max(1, std::min(s, std::max(1, K / kWgradChunk)));
+        *chunk = (K + s - 1) / s;
+        *chunk = (*chunk + kWgradChunk - 1) / kWgradChunk * kWgradChunk;
+        return (K + *chunk - 1) / *chunk;
+    };
+    // A one-pass epoch gives the same bits with and without the static scratch,
+    // so where the split tiles' partials do not fit it, every call of the plan
+    // takes the direct tiles, whose partials are a sixteenth.
+    if (split && one_pass_fits(p)) {
+        size_t floats = 0;
+        for (int k = 0, chunk; k < T; ++k)
+            floats += size_t(splits_of(k, &chunk)) * n.neurons[first + k + 1] * (n.neurons[first + k] + 1);
+        if (floats > static_partial_floats(epoch_blocks(p))) {
+            split = has256 = false;
+            total_tiles = count_tiles();
+        }
+    }
+    g.wa.direct = split ? 2 : direct ? 1 : 0;
     g.wa.block_begin[0] = 0;
     g.ra.accumulate = accumulate ? 1 : 0;
     g.ra.transitions = T;
@@ -666,14 +721,10 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     for (int k = 0; k < T; ++k) {
         const int t = first + k;
         const int M = n.neurons[t + 1], N = n.neurons[t];
-        int s = external_splits[t];
-        if (!s) {
+        int chunk = 0;
+        const int s = splits_of(k, &chunk);
+        if (!external_splits[t]) {
             const int tiles = thin(k) ? 1 : tiles_of(k);
-            s = thin(k) ? 2 * d.compute_units : tile_splits;
-            s = std::max(1, std::min(s, std::max(1, K / kWgradChunk)));
-            int chunk = (K + s - 1) / s;
-            chunk = (chunk + kWgradChunk - 1) / kWgradChunk * kWgradChunk;
-            s = (K + chunk - 1) / chunk;
             g.wa.M[w] = M;
             g.wa.N[w] = N;
             g.wa.K[w] = K;
@@ -1737,11 +1788,11 @@ int cpde_epoch_matching_static(cpde_plan* plan, const float* target, int target_
                 "the no-allocation epoch needs a plan whose one-pass epoch applies (network-fused kernels, the "
                 "chunk's workgroups resident on the device together)");
         const int blocks = epoch_blocks(*plan);
-        const size_t record_bytes = (sizeof(CostStats) * size_t(blocks) + 255) / 256 * 256;
+        const size_t record_bytes = static_record_bytes(blocks);
         require(record_bytes < size_t(CPDE_STATIC_SCRATCH_BYTES), "cost records beyond the static scratch");
         CostStats* records = reinterpret_cast<CostStats*>(d.static_scratch);
         const PartialSpace space{reinterpret_cast<float*>(d.static_scratch + record_bytes),
-                                 (size_t(CPDE_STATIC_SCRATCH_BYTES) - record_bytes) / sizeof(float)};
+                                 static_partial_floats(blocks)};
         MatchArgsHost m{target, target_rows, weights, records, target_width, weight_samples, offset, valid,
                         collect != 0};
         one_pass_epoch(*plan, plan->fused->network_epoch, &m, records, cost_index, accumulate != 0, space);

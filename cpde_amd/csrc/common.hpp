@@ -183,11 +183,13 @@ struct WgradArgs {
     const float* Y[kMaxTransitions];
     float* partial[kMaxTransitions];
     int M[kMaxTransitions], N[kMaxTransitions], kchunk[kMaxTransitions];
-    int tile[kMaxTransitions];  // 128, or 64 when both sides are at most 64
+    int tile[kMaxTransitions];  // 256, 128 or 64
     int block_begin[kMaxTransitions + 1];
     int K[kMaxTransitions], R[kMaxTransitions];  // columns and rows per point of each entry's pass
     int transitions;
-    int direct;  // 1: 64x64 tiles fed straight from global memory (wgrad_direct_kernel)
+    // 1: 64x64 tiles fed straight from global memory (wgrad_direct_kernel);
+    // 2: those, and split-product tiles where tile is 128 or 256 (wgrad_split_kernel)
+    int direct;
 };
 // The scalar cost graph's evaluation (cost_graph::execute) as one lane runs it.
 struct GraphLaunch {

@@ -457,8 +457,8 @@ __device__ __forceinline__ void split_planes(const float (&x)[8], uintx4 (&plane
     }
 }
 
-// One 64 WM x 64 WN tile of A B^T over k in [kbegin, kend): four waves, each a
-// 64 x 64 block of sixteen 16 x 16 products.  An operand's rows pass through LDS
+// A tile of A B^T over k in [kbegin, kend), each wave a block of 64 rows of A
+// (four 16 x 16 products high).  An operand's rows pass through LDS
 // in steps of 32 columns of k, split on the way in, laid out as the matrix
 // instruction reads them: for 16 rows, three planes of 64 lanes x 16 bytes
 // (lane (q, j): row j, k = 8q .. 8q + 7), so the reads are contiguous; 16 rows
@@ -473,59 +473,89 @@ constexpr int kSpRows16 = 3 * 1024 + 16;  // bytes of 16 rows of one 32-column s
 constexpr int sp_lds_bytes(int rows) { return rows / 16 * kSpRows16; }
 
 // A thread's share of ROWS x 32 elements among the workgroup's 256 threads:
-// chunks of eight k's, of rows 16 apart (K_MAJOR) or adjacent (not).
-template <int ROWS, bool K_MAJOR, bool VEC>
+// chunks of eight k's, of rows 16 apart (K_MAJOR) or adjacent (not).  Addresses
+// are a uniform base and a 32-bit offset within the tile.  Rows past the
+// operand's last repeat it (their products are not stored); k's past kend are
+// zero.
+template <int ROWS, bool K_MAJOR, bool VEC, int THREADS = 256>
 struct SplitStage {
-    static constexpr int kChunks = ROWS / 64;
-    static_assert(ROWS % 64 == 0 && (K_MAJOR || kChunks <= 2), "whole chunks per thread");
+    static constexpr int kChunks = ROWS * 4 / THREADS;
+    static constexpr int kGroups = ROWS / kChunks;  // threads side by side along the rows (not K_MAJOR)
+    static_assert(kChunks * THREADS == ROWS * 4 && (K_MAJOR || kChunks <= 2), "whole chunks per thread");
+    const float* base;  // the tile's first row (K_MAJOR) or the operand
+    int ld, kq;         // kq: the thread's first k within a step
+    unsigned offset[kChunks];
     float raw[kChunks][8];
 
-    __device__ __forceinline__ void load(const float* __restrict__ p, int ld, int rows, int row0, int k0, int kend,
-                                         int tid) {
+    __device__ __forceinline__ SplitStage(const float* __restrict__ p, int ld_, int rows, int row0, int tid) : ld(ld_) {
         if constexpr (K_MAJOR) {
+            base = p + size_t(ld) * row0;
+            kq = 8 * ((tid >> 4) & 3);
+#pragma unroll
+            for (int c = 0; c < kChunks; ++c)
+                offset[c] =
+                    unsigned(ld) * unsigned(min(16 * (tid >> 6) + THREADS / 4 * c + (tid & 15), rows - 1 - row0)) + kq;
+        } else {
+            base = p;
+            kq = 8 * (tid / kGroups);
+#pragma unroll
+            for (int c = 0; c < kChunks; ++c)  // float2 loads start at an even row
+                offset[c] = unsigned(min(row0 + kChunks * (tid % kGroups) + c, rows - (VEC ? kChunks - c : 1))) +
+                            unsigned(ld) * unsigned(kq);
+        }
+    }
+
+    // 32 columns from k0
+    __device__ __forceinline__ void load(int k0) {
+        if constexpr (K_MAJOR) {
+            const float* src = base + k0;
 #pragma unroll
             for (int c = 0; c < kChunks; ++c) {
-                const int s = tid + 256 * c, row = row0 + (s >> 6) * 16 + (s & 15), k = k0 + 8 * ((s >> 4) & 3);
-                const float* src = p + size_t(ld) * row + k;
                 if constexpr (VEC) {
-                    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-                    const floatx4 lo = row < rows && k < kend ? *reinterpret_cast<const floatx4*>(src) : zero;
-                    const floatx4 hi = row < rows && k + 4 < kend ? *reinterpret_cast<const floatx4*>(src + 4) : zero;
+                    const floatx4 a = *reinterpret_cast<const floatx4*>(src + offset[c]);
+                    const floatx4 b = *reinterpret_cast<const floatx4*>(src + offset[c] + 4);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        raw[c][i] = lo[i];
-                        raw[c][4 + i] = hi[i];
+                        raw[c][i] = a[i];
+                        raw[c][4 + i] = b[i];
                     }
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) raw[c][i] = row < rows && k + i < kend ? src[i] : 0.0f;
+                    for (int i = 0; i < 8; ++i) raw[c][i] = src[offset[c] + i];
                 }
             }
         } else {
-            const int row = row0 + kChunks * (tid & 63), k = k0 + 8 * (tid >> 6);
-            const float* src = p + row + size_t(ld) * k;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
+                const float* src = base + size_t(ld) * (k0 + i);
                 if constexpr (kChunks == 2 && VEC) {
-                    floatx2 v = {0.0f, 0.0f};
-                    if (k + i < kend && row < rows) v = *reinterpret_cast<const floatx2*>(src + size_t(ld) * i);
+                    const floatx2 v = *reinterpret_cast<const floatx2*>(src + offset[0]);
                     raw[0][i] = v[0];
                     raw[1][i] = v[1];
                 } else {
 #pragma unroll
-                    for (int r = 0; r < kChunks; ++r)
-                        raw[r][i] = k + i < kend && row + r < rows ? src[size_t(ld) * i + r] : 0.0f;
+                    for (int r = 0; r < kChunks; ++r) raw[r][i] = src[offset[r]];
                 }
             }
         }
+    }
+    // the fewer than 32 left before kend
+    __device__ __forceinline__ void load_tail(int k0, int kend) {
+        const float* src = K_MAJOR ? base + k0 : base + size_t(ld) * k0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int c = 0; c < kChunks; ++c)
+                raw[c][i] = k0 + kq + i < kend ? src[offset[c] + (K_MAJOR ? unsigned(i) : unsigned(ld) * unsigned(i))]
+                                               : 0.0f;
     }
 
     __device__ __forceinline__ void store(unsigned char* lds, int tid) const {
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
-            const int s = tid + 256 * c;
-            const int row = K_MAJOR ? (s >> 6) * 16 + (s & 15) : kChunks * (tid & 63) + c;
-            const int q = K_MAJOR ? (s >> 4) & 3 : tid >> 6;
+            const int s = tid + THREADS * c;
+            const int row = K_MAJOR ? (s >> 6) * 16 + (s & 15) : kChunks * (tid % kGroups) + c;
+            const int q = K_MAJOR ? (s >> 4) & 3 : tid / kGroups;
             uintx4 plane[3];
             split_planes(raw[c], plane);
             unsigned char* dst = lds + (row >> 4) * kSpRows16 + q * 256 + (row & 15) * 16;
@@ -535,43 +565,101 @@ struct SplitStage {
     }
 };
 
-// The accumulators of a wave's 64 x 64 block: big + small is the product;
-// register v of lane (q, j) of (a, b) is row 16a + 4q + v, column 16b + j.
+// The sums of a wave's 64 x 16 NB block: register v of lane (q, j) of (a, b) is
+// row 16a + 4q + v, column 16b + j.
+template <int NB>
 struct SplitBlock {
-    floatx4 big[4][4], small[4][4];
+    floatx4 sum[4][NB];
     __device__ __forceinline__ void clear() {
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) big[a][b] = small[a][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int b = 0; b < NB; ++b) sum[a][b] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     }
 };
 
-// One step's products from the staged rows (A: 4 x 16 rows at la, B at lb).
-__device__ __forceinline__ void split_products(SplitBlock& c, const unsigned char* la, const unsigned char* lb,
+// One step's products from the staged rows (A: 4 x 16 rows at la, B: NB x 16 at
+// lb), XS of the four A blocks at a time (with two, the registers suffice for
+// the wider waves, and B is read twice).
+template <int NB>
+__device__ __forceinline__ void split_products(SplitBlock<NB>& c, const unsigned char* la, const unsigned char* lb,
                                                int lane) {
-    bf16x8 a[4][3];
+    constexpr int XS = NB > 4 ? 2 : 4, YS = 4 / XS;  // four independent chains between dependent products
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x0 = 0; x0 < 4; x0 += XS) {
+        bf16x8 a[XS][3];
 #pragma unroll
-        for (int s = 0; s < 3; ++s)
-            a[x][s] = *reinterpret_cast<const bf16x8*>(la + x * kSpRows16 + 1024 * s + 16 * lane);
+        for (int x = 0; x < XS; ++x)
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
-        bf16x8 b[3];
+            for (int s = 0; s < 3; ++s)
+                a[x][s] = *reinterpret_cast<const bf16x8*>(la + (x0 + x) * kSpRows16 + 1024 * s + 16 * lane);
 #pragma unroll
-        for (int s = 0; s < 3; ++s) b[s] = *reinterpret_cast<const bf16x8*>(lb + y * kSpRows16 + 1024 * s + 16 * lane);
-        // four independent accumulators between dependent products
-#define CPDE_SPLIT_TERM(acc, i, k) \
-    _Pragma("unroll") for (int x = 0; x < 4; ++x) \
-        c.acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x][i], b[k], c.acc[x][y], 0, 0, 0);
-        CPDE_SPLIT_TERM(small, 0, 2)
-        CPDE_SPLIT_TERM(big, 0, 0)
-        CPDE_SPLIT_TERM(small, 2, 0)
-        CPDE_SPLIT_TERM(small, 1, 1)
-        CPDE_SPLIT_TERM(small, 0, 1)
-        CPDE_SPLIT_TERM(small, 1, 0)
-#undef CPDE_SPLIT_TERM
+        for (int y0 = 0; y0 < NB; y0 += YS) {
+            bf16x8 b[YS][3];
+#pragma unroll
+            for (int y = 0; y < YS; ++y)
+#pragma unroll
+                for (int s = 0; s < 3; ++s)
+                    b[y][s] = *reinterpret_cast<const bf16x8*>(lb + (y0 + y) * kSpRows16 + 1024 * s + 16 * lane);
+            floatx4 t[XS][YS];
+#pragma unroll
+            for (int x = 0; x < XS; ++x)
+#pragma unroll
+                for (int y = 0; y < YS; ++y) t[x][y] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            constexpr int kTerm[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};  // the small terms first
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+#pragma unroll
+                for (int x = 0; x < XS; ++x)
+#pragma unroll
+                    for (int y = 0; y < YS; ++y)
+                        t[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x][kTerm[k][0]], b[y][kTerm[k][1]], t[x][y],
+                                                                          0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < XS; ++x)
+#pragma unroll
+                for (int y = 0; y < YS; ++y) c.sum[x0 + x][y0 + y] += t[x][y];
+            if constexpr (NB > 4) __builtin_amdgcn_sched_barrier(0);  // holds later reads back: their registers
+        }
+    }
+}
+
+// The tile's sums over k in [kbegin, kend): per step, the staged values are
+// converted and stored, and the next step's loads fly during its products.  The
+// columns left over from whole steps come last, outside the loop (inside, their
+// guarded addresses took the loop's registers).
+template <int NB, class SA, class SB>
+__device__ __forceinline__ void split_accumulate(SplitBlock<NB>& c, SA& sa, SB& sb, int kbegin, int kend,
+                                                 unsigned char* la, unsigned char* lb, int row_a, int row_b) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const unsigned char* const wa = la + sp_lds_bytes(row_a);
+    const unsigned char* const wb = lb + sp_lds_bytes(row_b);
+    const int whole = kbegin + (kend - kbegin) / 32 * 32;
+    c.clear();
+    if (kbegin < whole) {
+        sa.load(kbegin);
+        sb.load(kbegin);
+#pragma unroll 1
+        for (int k0 = kbegin; k0 < whole; k0 += 32) {
+            sa.store(la, tid);
+            sb.store(lb, tid);
+            __syncthreads();
+            if (k0 + 32 < whole) {
+                sa.load(k0 + 32);
+                sb.load(k0 + 32);
+            }
+            split_products(c, wa, wb, lane);
+            __syncthreads();
+        }
+    }
+    if (whole < kend) {
+        sa.load_tail(whole, kend);
+        sb.load_tail(whole, kend);
+        sa.store(la, tid);
+        sb.store(lb, tid);
+        __syncthreads();
+        split_products(c, wa, wb, lane);
+        __syncthreads();
     }
 }
 
@@ -595,25 +683,13 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K,
     const int tiles_m = (M + TM - 1) / TM;
     const int block = xcd_grouped(int(blockIdx.x), int(gridDim.x));  // the tiles of the same B rows on one XCD
     const int m0 = (block % tiles_m) * TM, n0 = (block / tiles_m) * TN;
-    SplitStage<TM, A_K, VEC> sa;
-    SplitStage<TN, true, VEC> sb;
-    auto load = [&](int k0) {
-        sa.load(A, lda, M, m0, k0, K, tid);
-        sb.load(B, ldb, N, n0, k0, K, tid);
-    };
-    SplitBlock c;
-    c.clear();
-    load(0);
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        sa.store(la, tid);
-        sb.store(lb, tid);
-        __syncthreads();
-        if (k0 + 32 < K) load(k0 + 32);
-        split_products(c, la + (wave % WM) * sp_lds_bytes(64), lb + (wave / WM) * sp_lds_bytes(64), lane);
-        __syncthreads();
-    }
+    SplitStage<TM, A_K, VEC> sa(A, lda, M, m0, tid);
+    SplitStage<TN, true, VEC> sb(B, ldb, N, n0, tid);
+    SplitBlock<4> c;
+    split_accumulate(c, sa, sb, 0, K, la, lb, 64 * (wave % WM), 64 * (wave / WM));
     const int q = lane >> 4, j = lane & 15;
     const int mw = m0 + 64 * (wave % WM) + 4 * q, nw = n0 + 64 * (wave / WM) + j;
+    const bool quads = (M | ldc) % 4 == 0 && ((reinterpret_cast<size_t>(C) | reinterpret_cast<size_t>(bias)) & 15) == 0;
 #pragma unroll
     for (int y = 0; y < 4; ++y) {
         const int n = nw + 16 * y;
@@ -622,9 +698,9 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K,
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
             const int m = mw + 16 * x;
-            floatx4 v = c.big[x][y] + c.small[x][y];
+            floatx4 v = c.sum[x][y];
             float* dst = C + m + size_t(ldc) * n;
-            if (VEC && m + 4 <= M) {  // ldc is a multiple of 4 with the A operand's extent
+            if (quads && m + 4 <= M) {
                 if (add) v += *reinterpret_cast<const floatx4*>(bias + m);
                 *reinterpret_cast<floatx4*>(dst) = v;
             } else {
@@ -1247,6 +1323,64 @@ __device__ __forceinline__ void wgrad_direct_tile(const WgradArgs& a, int t, int
     }
 }
 
+// Weight-gradient tile of TILE x TILE (128 or 256) on the split products, for
+// transitions wider than 64 on both sides: the workgroup converts each value of
+// its split once for the tile's rows or columns.  128: four waves of 64 x 64,
+// two workgroups per CU; 256: eight waves of 64 x 128, one workgroup per CU,
+// each stack read once for widths up to 256.  The split's columns come in steps of 32; the bias
+// (n-tile 0) as in the direct tiles, eight loads in flight per lane.
+template <int TILE, bool VEC>
+__device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, int t, int local, unsigned char* lds) {
+    constexpr int THREADS = 2 * TILE, WR = TILE / 64, NB = TILE / 32;  // waves along the rows; 16-column blocks of a wave
+    const int M = a.M[t], N = a.N[t], K = a.K[t], R = a.R[t];
+    const int tiles_m = (M + TILE - 1) / TILE, tiles_n = (N + TILE - 1) / TILE;
+    const int tile = local % (tiles_m * tiles_n), split = local / (tiles_m * tiles_n);
+    const int m0 = (tile % tiles_m) * TILE, n0 = (tile / tiles_m) * TILE;
+    const int kbegin = split * a.kchunk[t], kend = min(K, kbegin + a.kchunk[t]);
+    const float* __restrict__ G = a.G[t];
+    const float* __restrict__ Y = a.Y[t];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int mw = 64 * (wave % WR), nw = 16 * NB * (wave / WR);
+    unsigned char* const la = lds;
+    unsigned char* const lb = lds + sp_lds_bytes(TILE);
+    SplitStage<TILE, false, VEC, THREADS> sa(G, M, M, m0, tid), sb(Y, N, N, n0, tid);
+    SplitBlock<NB> c;
+    split_accumulate(c, sa, sb, kbegin, kend, la, lb, mw, nw);
+    float* P = a.partial[t] + size_t(split) * M * (N + 1);
+    if (n0 == 0) {
+        const int row = tid % TILE, half = tid / TILE;
+        float sum = 0.0f;
+        if (m0 + row < M) {
+            constexpr int U = 8;
+            for (int k = (kbegin + R - 1) / R * R + R * half; k < kend; k += 2 * R * U) {
+                float v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    v[u] = G[size_t(min(k + 2 * R * u, kend - 1)) * M + m0 + row];
+#pragma unroll
+                for (int u = 0; u < U; ++u) sum += k + 2 * R * u < kend ? v[u] : 0.0f;
+            }
+        }
+        float* halves = reinterpret_cast<float*>(lds);
+        halves[tid] = sum;
+        __syncthreads();
+        if (half == 0 && m0 + row < M) P[size_t(m0 + row) * (N + 1) + N] = halves[row] + halves[TILE + row];
+    }
+    const int q = lane >> 4, j = lane & 15;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int m = m0 + mw + 16 * x + 4 * q + v;
+            if (m >= M) continue;
+#pragma unroll
+            for (int y = 0; y < NB; ++y) {
+                const int n = n0 + nw + 16 * y + j;
+                if (n < N) P[size_t(m) * (N + 1) + n] = c.sum[x][y][v];
+            }
+        }
+}
+
 // Direct tiles and the thin transitions' roles in one launch (33 KB of LDS
 // per workgroup).
 #ifndef CPDE_WD_MIN_BLOCKS
@@ -1263,10 +1397,70 @@ __global__ __launch_bounds__(256, CPDE_WD_MIN_BLOCKS) void wgrad_direct_kernel(W
     else wgrad_direct_tile<false>(a, t, local, lds);
 }
 
+// The same with split tiles where tile[t] is 128 (49.4 KB of LDS, two
+// workgroups per CU).
+__global__ __launch_bounds__(256, 2) void wgrad_split_kernel(WgradArgs a) {
+    constexpr int kBytes = sp_lds_bytes(256) > 4 * kWdLds ? sp_lds_bytes(256) : 4 * kWdLds;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kBytes];
+    float* const floats = reinterpret_cast<float*>(lds);
+    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
+    const int t = group_of(a.block_begin, a.transitions, b);
+    const int local = b - a.block_begin[t];
+    const bool vec = a.M[t] % 4 == 0 && a.N[t] % 4 == 0;
+    if (a.tile[t] == 128) {
+        if (vec) wgrad_split_tile<128, true>(a, t, local, lds);
+        else wgrad_split_tile<128, false>(a, t, local, lds);
+    } else if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin(a, t, local, floats);
+    else if (vec) wgrad_direct_tile<true>(a, t, local, floats);
+    else wgrad_direct_tile<false>(a, t, local, floats);
+}
+
+// Split tiles of 256 x 256 (98.8 KB of LDS).
+template <bool VEC>
+__global__ __launch_bounds__(512, 2) void wgrad_split256_kernel(WgradArgs a) {
+    __shared__ __attribute__((aligned(16))) unsigned char lds[sp_lds_bytes(512)];
+    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
+    const int t = group_of(a.block_begin, a.transitions, b);
+    wgrad_split_tile<256, VEC>(a, t, b - a.block_begin[t], lds);
+}
+
+// The entries of a whose tile is 256 (or is not), renumbered.
+static WgradArgs wgrad_tiles(const WgradArgs& a, bool tile256) {
+    WgradArgs r{};
+    r.direct = a.direct;
+    for (int k = 0; k < a.transitions; ++k) {
+        if ((a.tile[k] == 256) != tile256) continue;
+        const int w = r.transitions++;
+        r.G[w] = a.G[k];
+        r.Y[w] = a.Y[k];
+        r.partial[w] = a.partial[k];
+        r.M[w] = a.M[k];
+        r.N[w] = a.N[k];
+        r.K[w] = a.K[k];
+        r.R[w] = a.R[k];
+        r.kchunk[w] = a.kchunk[k];
+        r.tile[w] = a.tile[k];
+        r.block_begin[w + 1] = r.block_begin[w] + a.block_begin[k + 1] - a.block_begin[k];
+    }
+    return r;
+}
+
 void launch_wgrad_grouped(Device& d, const WgradArgs& a, double flops) {
     TraceScope trace(d, kTraceWgrad, flops);
-    if (a.direct) hipLaunchKernelGGL(wgrad_direct_kernel, a.block_begin[a.transitions], 256, 0, d.stream, a);
-    else hipLaunchKernelGGL(wgrad_grouped_kernel, a.block_begin[a.transitions], 256, 0, d.stream, a);
+    if (a.direct == 2) {
+        // 256 x 256 tiles have workgroups of 512 and go out on their own
+        const WgradArgs wide = wgrad_tiles(a, true), rest = wgrad_tiles(a, false);
+        bool vec = true;
+        for (int k = 0; k < wide.transitions; ++k) vec = vec && wide.M[k] % 4 == 0 && wide.N[k] % 4 == 0;
+        if (wide.transitions)
+            hipLaunchKernelGGL(vec ? wgrad_split256_kernel<true> : wgrad_split256_kernel<false>,
+                               wide.block_begin[wide.transitions], 512, 0, d.stream, wide);
+        if (rest.transitions)
+            hipLaunchKernelGGL(wgrad_split_kernel, rest.block_begin[rest.transitions], 256, 0, d.stream, rest);
+    } else if (a.direct)
+        hipLaunchKernelGGL(wgrad_direct_kernel, a.block_begin[a.transitions], 256, 0, d.stream, a);
+    else
+        hipLaunchKernelGGL(wgrad_grouped_kernel, a.block_begin[a.transitions], 256, 0, d.stream, a);
     HIP_CHECK(hipGetLastError());
 }
 
