@@ -300,7 +300,7 @@ struct NetArgsHost {
     const float* X;
     float* partial_in;
     float* partial_out;
-    float* WT[32];
+    void* WS[32];
     float* partial_hidden[32];
     int block_offset, block_count;  // the pass's workgroups in the launch (count 0: the whole grid)
 };
@@ -353,8 +353,11 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // CUs it was slower (order 4, 365 workgroups: 0.0700 -> 0.0742).
     if (width > 0 && rows <= 16 && npb > 1 && !value_leaf && (width + npb - 1) / npb <= compute_units)
         t.net_threads = 512;
+    // Two points of layers wider than 128 leave room for one workgroup per CU:
+    // eight waves (2->256^4->1, order 6: 74.5 -> 68.1 ms per epoch).
+    if (t.alias && *std::max_element(neurons.begin(), neurons.end()) > 128) t.net_threads = 512;
     t.net_threads = env_int("CPDE_NET_THREADS", t.net_threads) == 512 ? 512 : 256;
-    // The waves of a workgroup share a layer's products by output tile.  Where
+    // The waves of a workgroup share a layer's fp32 products by output tile.  Where
     // 32x32 tiles of the narrowest hidden layer are fewer than the waves (a
     // 128-wide layer in eight waves, a 64-wide one in four), 16-column tiles
     // keep every wave busy.  2->128^4->1 over 729 points, ms per epoch with
@@ -377,12 +380,16 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // none: order 5 (21 rows) 0.0936 / 0.0904, order 6 (28 rows) 0.1036 /
     // 0.0992; orders 1-4, several points per workgroup, within 0.3 %).
     const bool whole = rows > 32 || (rows > 16 && t.net_points_per_block == 1);
-    t.max_split = std::max(1, env_int("CPDE_NET_SPLIT", whole ? 1 : t.max_split));
+    // (Where whole compositions leave three lanes of four idle the mirror split
+    // still pays: 2->32^2->1 at order 6 over 40 points 21.2 -> 20.7 us.)
+    const int widest = *std::max_element(neurons.begin(), neurons.end());
+    const bool sparse = rows > 16 && 4 * t.net_points_per_block * widest <= t.net_threads;
+    t.max_split = std::max(1, env_int("CPDE_NET_SPLIT", whole && !sparse ? 1 : t.max_split));
     t.max_split_adjoint = std::max(1, env_int("CPDE_NET_SPLIT_ADJOINT", t.max_split_adjoint));
     t.forward_blocks = std::max(1, env_int("CPDE_NET_FWD_OCC", t.forward_blocks));
     t.backward_blocks = std::max(1, env_int("CPDE_NET_BWD_OCC", t.backward_blocks));
-    t.col_tile = env_int("CPDE_NET_COLTILE", t.col_tile);
     t.alias = env_int("CPDE_NET_ALIAS", t.alias);
+    t.col_tile = env_int("CPDE_NET_COLTILE", t.col_tile);
     // Paired neuron blocks in the 16-column products (weight operands as
     // float2, one LDS operand read per two products), on wherever a layer's
     // width is a multiple of 32 per wave.  Measured, ms per epoch against the
@@ -393,11 +400,6 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // Diagnostics: clock stamps of the one-pass epoch's phases, written over
     // the output stack (cpde_amd/stamps.py reads them back).
     t.stamps = env_int("CPDE_PHASE_STAMPS", 0) ? 1 : 0;
-    // One-pass epochs: wave priority by dispatch round (tier_priority in the
-    // generated source; 0 turns it off).  It acts only where a launch has more
-    // workgroups than CUs.
-    t.tier_prio = env_int("CPDE_NET_TIER_PRIO", 125);
-    t.tier_cus = compute_units;
     // Hidden weight-gradient partials from the network backward itself, on
     // request (CPDE_INKERNEL_WGRAD=1; hidden widths that are multiples of 16).
     // Measured on the Poisson graph epoch, whose 256-point one-row boundary
@@ -474,7 +476,7 @@ static NetArgsHost net_args(const Plan& p) {
     NetArgsHost a{};
     for (int t = 0; t + 1 < n.layers; ++t) {
         a.W[t] = n.state[0][t];
-        a.WT[t] = n.wt[t];
+        a.WS[t] = n.ws[t];
     }
     for (int l = 0; l < n.layers; ++l) {
         a.Z[l] = n.z[l];
@@ -522,6 +524,23 @@ static GradientPlan network_gradients(Plan& p, int blocks, bool accumulate, cons
 // Mode of the fused path: CPDE_FUSED=2 (default) network-fused, 1 layer-fused.
 static bool network_mode() { return env_int("CPDE_FUSED", 2) >= 2; }
 
+// Rewrite the product operands of every hidden transition from the weights
+// (one launch).
+static void refresh_operands(Net& n) {
+    std::vector<const float*> W;
+    std::vector<void*> WS;
+    std::vector<int> ni, no;
+    for (int t = 1; t + 2 < n.layers; ++t) {
+        if (!n.ws[t]) continue;
+        W.push_back(n.state[0][t]);
+        WS.push_back(n.ws[t]);
+        ni.push_back(n.neurons[t]);
+        no.push_back(n.neurons[t + 1]);
+    }
+    if (!W.empty()) launch_weight_operands(*n.dev, W.data(), WS.data(), ni.data(), no.data(), int(W.size()), n.split);
+    n.ws_current = true;
+}
+
 static void fused_forward(Plan& p) {
     Net& n = *p.net;
     Device& d = *n.dev;
@@ -530,6 +549,7 @@ static void fused_forward(Plan& p) {
     int width = p.width;
     const double cols = double(p.columns());
     if (p.network) {
+        if (n.split && (!n.ws_current || n.weights_out)) refresh_operands(n);
         NetArgsHost a = net_args(p);
         void* args[] = {&a, &width};
         double flops = 0;
@@ -537,7 +557,7 @@ static void fused_forward(Plan& p) {
         TraceScope trace(d, kTraceNetworkForward, flops);
         launch_module(d, fm.network_forward, unsigned((width + fm.net_points_per_block - 1) / fm.net_points_per_block),
                       1, args, unsigned(fm.net_threads));
-        n.wt_current = true;  // written by the forward's side job
+        n.ws_current = true;  // fp32 products: written by the forward's side job
         return;
     }
     {
@@ -917,7 +937,7 @@ static void flush_if_reads(Device& d, const CostStats* records, int slot = -1) {
 // (launch_rprop does the same after its own launch).
 static void rprop_done(Net& n) {
     for (auto& act : n.active) act = act == 1 ? 2 : 1;
-    n.wt_current = true;
+    n.ws_current = true;
 }
 
 // Host mirror of the one-pass epoch's matching arguments (fused.hip.in MatchArgs).
@@ -948,22 +968,6 @@ static int epoch_blocks(const Plan& p) {
 // CPDE_ONE_PASS=0 forces the separate launches (same kernels otherwise).
 static bool one_pass_fits(const Plan& p) {
     return env_int("CPDE_ONE_PASS", 1) && p.fused && p.network && epoch_blocks(p) <= 4 * p.net->dev->compute_units;
-}
-
-// Rewrite the row-major weight copies of every hidden transition from the
-// weights (one launch).
-static void refresh_wt(Net& n) {
-    std::vector<const float*> W;
-    std::vector<float*> WT;
-    std::vector<int> ni, no;
-    for (int t = 1; t + 2 < n.layers; ++t) {
-        W.push_back(n.state[0][t]);
-        WT.push_back(n.wt[t]);
-        ni.push_back(n.neurons[t]);
-        no.push_back(n.neurons[t + 1]);
-    }
-    if (!W.empty()) launch_transpose(*n.dev, W.data(), WT.data(), ni.data(), no.data(), int(W.size()));
-    n.wt_current = true;
 }
 
 // The per-workgroup cost records of a one-pass epoch.
@@ -1178,7 +1182,7 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
     // the backward half reads the row-major weight copies of every hidden
     // transition, which no workgroup of the same launch may still be writing;
     // RPROP and Adam keep them current between epochs
-    if (!n.wt_current) refresh_wt(n);
+    if (!n.ws_current) refresh_operands(n);
     void* args[] = {&a, cost_args, &width};
     double flops = 0;
     for (int t = 0; t + 1 < L; ++t) flops += 2.0 * n.neurons[t] * n.neurons[t + 1] * cols;
@@ -1417,7 +1421,8 @@ int cpde_net_create(cpde_device* dev, int layers, const int* neurons, const int*
         n->linear.assign(linear, linear + layers);
         const int T = layers - 1;
         for (auto& s : n->state) s.assign(T, nullptr);
-        n->wt.assign(T, nullptr);
+        n->split = split_products(n->neurons);
+        n->ws.assign(T, nullptr);
         n->active.assign(T, 1);
         n->z.assign(layers, nullptr);
         n->y.assign(layers, nullptr);
@@ -1426,7 +1431,13 @@ int cpde_net_create(cpde_device* dev, int layers, const int* neurons, const int*
         for (int t = 0; t < T; ++t) {
             const size_t count = n->param_count(t);
             for (int b = 0; b < 4; ++b) HIP_CHECK(hipMalloc(&n->state[b][t], count * sizeof(float)));
-            HIP_CHECK(hipMalloc(&n->wt[t], size_t(n->neurons[t]) * n->neurons[t + 1] * sizeof(float)));
+// the widths that the network-fused kernels take
+            if (t > 0 && t + 1 < T && n->neurons[t] <= 256 && n->neurons[t + 1] <= 256) {
+                const size_t words = n->split ? weight_operands(n->neurons[t], n->neurons[t + 1]) / 2
+                                              : size_t(n->neurons[t]) * n->neurons[t + 1];
+                HIP_CHECK(hipMalloc(&n->ws[t], words * sizeof(float)));
+                if (n->split) launch_fill(*dev, static_cast<float*>(n->ws[t]), words, 0.0f);  // the padding stays zero
+            }
             if (initial && initial[t])
                 HIP_CHECK(hipMemcpyAsync(n->state[0][t], initial[t], count * sizeof(float), hipMemcpyHostToDevice,
                                          dev->stream));
@@ -1456,7 +1467,7 @@ int cpde_net_destroy(cpde_net* net) {
         ++net->dev->layout;
         for (auto& s : net->state)
             for (float* p : s) (void)hipFree(p);
-        for (float* p : net->wt) (void)hipFree(p);
+        for (void* p : net->ws) (void)hipFree(p);
         for (auto* v : {&net->z, &net->y, &net->g})
             for (float* p : *v) (void)hipFree(p);
         (void)hipFree(net->partials);
@@ -1468,7 +1479,10 @@ int cpde_net_state(cpde_net* net, int transition, int buffer, float** device_ptr
     return guarded([&] {
         flush_reduce(*net->dev);
         require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
-        if (buffer == 0) net->wt_current = false;  // the caller may write the weights
+        if (buffer == 0) {  // the caller may write the weights
+            net->ws_current = false;
+            net->weights_out = true;
+        }
         if (device_ptr) *device_ptr = net->state[buffer][transition];
         if (count) *count = net->param_count(transition);
     });
@@ -1944,7 +1958,7 @@ static int issue_update(cpde_device* dev, int costs, int layers, int with_graph,
         // with its own test the launch reads no gradient totals
         const UpdateGuard guard{dev->cost_totals, costs, fresh, test ? nullptr : dev->grad_totals, test ? 0 : layers,
                                 with_graph ? dev->graph_summary : nullptr};
-        const bool wt_current = net->wt_current;
+        const bool ws_current = net->ws_current;
         if (method == 0) {
             launch_rprop(*dev, *net, &guard, &copy, test);
             rprop_done(*net);  // in expectation; cpde_update_resolve switches back if the rule rejects the epoch
@@ -1952,7 +1966,7 @@ static int issue_update(cpde_device* dev, int costs, int layers, int with_graph,
             launch_adam(*dev, *net, step, lr, &guard, &copy, test);
         }
         HIP_CHECK(hipEventRecord(dev->copied, dev->stream));
-        dev->issued = Device::IssuedUpdate{true, net, costs, layers, with_graph != 0, method == 0, wt_current, fresh};
+        dev->issued = Device::IssuedUpdate{true, net, costs, layers, with_graph != 0, method == 0, ws_current, fresh};
     });
 }
 
@@ -1987,7 +2001,7 @@ int cpde_update_resolve(cpde_device* dev, cpde_cost_stats* cost_out, cpde_gradie
         *updated = update_accepted(guard) ? 1 : 0;
         if (!*updated) {  // the update did not apply: RPROP's buffers switch back
             if (u.rprop) rprop_done(*u.net);
-            u.net->wt_current = u.wt_current;
+            u.net->ws_current = u.ws_current;
         }
     });
 }
@@ -2274,7 +2288,7 @@ int cpde_capture_begin(cpde_device* dev) {
 static void abandon_capture(Device& d) {
     for (auto& c : d.capture_nets) {
         c.net->active = c.active;
-        c.net->wt_current = false;
+        c.net->ws_current = false;
     }
     d.capture_nets.clear();
 }
@@ -2316,7 +2330,7 @@ int cpde_capture_end(cpde_device* dev, int keep, cpde_replay** out) {
             (void)hipGraphExecDestroy(exec);
             for (auto& c : r->nets) {
                 c.net->active = c.before;
-                c.net->wt_current = false;
+                c.net->ws_current = false;
             }
             HIP_CHECK(launched);
         }
@@ -2336,7 +2350,7 @@ int cpde_replay_launch(cpde_replay* replay) {
         }
         flush_reduce(d);
         for (const auto& c : replay->nets)
-            if (!c.net->wt_current) refresh_wt(*c.net);
+            if (!c.net->ws_current) refresh_operands(*c.net);
         HIP_CHECK(hipGraphLaunch(replay->exec, d.stream));
         for (const auto& c : replay->nets) c.net->active = c.after;
     });

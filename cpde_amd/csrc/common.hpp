@@ -103,13 +103,18 @@ struct Net {
     // Per transition t: four state buffers of n_{t+1} x (n_t+1) floats.
     std::vector<float*> state[4];
     std::vector<int> active;  // 1 or 2 per transition
-    // Per transition: n_t x n_{t+1} row-major copy of the weights (without the
-    // bias) for the backward's products.  Written by every network-fused
-    // forward and by the optimizer launches; the one-pass epoch transposes
-    // first only when wt_current is false (a new network, or the weights'
-    // device pointer handed out by cpde_net_state).
-    std::vector<float*> wt;
-    bool wt_current = false;
+    // Per hidden transition of a network that the network-fused kernels may
+    // take (else null): the weights as their products' operands.  With `split`,
+    // three bf16 planes in the matrix instruction's order, the forward's then the
+    // backward's (weight_operand in kernels.hip); otherwise the n_t x n_{t+1}
+    // row-major fp32 copy that the backward reads, which a separate forward also
+    // writes.  Written by the optimizer launches; the network kernels rewrite
+    // them first when ws_current is false (a new network, or the weights' device
+    // pointer handed out by cpde_net_state), and a separate forward on split
+    // operands whenever that pointer is out (weights_out), as its holder may
+    // write again.
+    std::vector<void*> ws;
+    bool split = false, ws_current = false, weights_out = false;
     // Stack arena shared by every plan of the network (contexts are views,
     // the reference's layer banks, cuda/cpde_engine.cuh:661-693).
     std::vector<float*> z, y, g;      // per layer
@@ -285,7 +290,7 @@ struct Device {
         int costs = 0, layers = 0;
         bool graph = false;
         bool rprop = true;        // RPROP (buffers switched in expectation), else Adam
-        bool wt_current = false;  // the network's before the issue
+        bool ws_current = false;  // the network's before the issue
         unsigned long long fresh = 0;
     } issued;
     // tracing
@@ -389,11 +394,10 @@ struct FusedTuning {
     int max_split_adjoint = 1;     // lanes per adjoint composition, at most
     int alias = 0;                 // network kernels: products write over their operand tile (one LDS tile)
     int forward_blocks = 2, backward_blocks = 2;  // blocks per CU the register budget must allow
-    int col_tile = 0;              // column tile of the network products: 16, 32, or 0 (chosen per shape)
+    int col_tile = 0;              // column tile of the fp32 network products: 16, 32, or 0 (chosen per shape)
+    int b_pairs = 1;               // fp32 16-column products: each wave takes 32-neuron blocks, B loaded as float2
     int scaled = 1;                // network kernels keep Taylor-scaled sigmoid stacks (row alpha / alpha!)
     int inkernel_wgrad = 0;        // network backward kernels write hidden weight-gradient partials themselves
-    int b_pairs = 1;               // 16-column products: each wave takes 32-neuron blocks, B loaded as float2
-    int tier_prio = 0, tier_cus = 256;  // one-pass epochs: wave priorities by dispatch round, and the CU count
     int stamps = 0;                // one-pass epochs write per-phase clock stamps over their output stack
 };
 // Whether the schema is closed under swapping variables 0 and 1 (the scaled
@@ -445,9 +449,16 @@ void launch_costs_begin(Device& d, int costs);
 // Statistics of `transitions` (<= kMaxTransitions) gradients into slots first_slot...
 void launch_grad_stats(Device& d, const float* const* g, const int* counts, int transitions, int first_slot);
 void launch_fill_grouped(Device& d, float* const* p, const int* counts, int buffers, float value);
-// WT[t][i + n_in*o] = W[t][o + n_out*i] for `count` blocks in one launch.
-void launch_transpose(Device& d, const float* const* W, float* const* WT, const int* n_in, const int* n_out,
-                      int count);
+// Whether a network's products run on split bf16 operands.
+bool split_products(const std::vector<int>& neurons);
+// bf16s of a transition's split weight operands (Net::ws).
+inline size_t weight_operands(int n_in, int n_out) {
+    const auto blocks = [](int n, int k) { return size_t((n + 15) / 16) * ((k + 31) / 32) * 3 * 512; };
+    return blocks(n_out, n_in) + blocks(n_in, n_out);
+}
+// The operands of `count` weight blocks in one launch (their padding is left alone).
+void launch_weight_operands(Device& d, const float* const* W, void* const* WS, const int* n_in, const int* n_out,
+                            int count, bool split);
 // Fixed-order sum of `blocks` per-workgroup cost records into cost slot cost_index.
 void launch_finish_cost(Device& d, const CostStats* partials, int blocks, int cost_index);
 // Zero the slots among [0, count) still marked fresh (before something reads them on the device).

@@ -668,6 +668,13 @@ static int forward_split_cap(const Tables& t, const FusedTuning& tuning) {
     return mirror_symmetric(t) ? std::min(tuning.max_split, 2) : 1;
 }
 
+// Whether a network's products run on split bf16 operands (fused.hip.in).
+bool split_products(const std::vector<int>& neurons) {
+    int widest = 0;
+    for (size_t l = 1; l + 1 < neurons.size(); ++l) widest = std::max(widest, neurons[l]);
+    return widest >= 128;
+}
+
 // Whether every hidden layer's forward and adjoint compositions have one lane
 // per (point, neuron) column (the row split of fused.hip.in's split_of is 1).
 static bool alias_tiles(const Tables& t, const std::vector<int>& neurons, const FusedTuning& tuning) {
@@ -682,7 +689,7 @@ static bool alias_tiles(const Tables& t, const std::vector<int>& neurons, const 
 // The network kernels' LDS tiles: the operand tile X and the product tile T,
 // which is X itself under CPDE_ALIAS_TILES.
 static std::string tile_declarations() {
-    return "    __shared__ __attribute__((aligned(16))) float X[kNNC * kS];\n"
+    return "    __shared__ __attribute__((aligned(16))) float X[kXF];\n"
            "#ifdef CPDE_ALIAS_TILES\n"
            "    float* const T = X;\n"
            "#else\n"
@@ -702,7 +709,7 @@ static void emit_prologue(std::ostream& o, const Tables& t, const std::vector<in
     o << "#define CPDE_NET_POINTS " << net_points_per_block << "\n";
     o << "#define CPDE_NET_THREADS " << tuning.net_threads << "\n";
     o << "#define CPDE_STRIDE " << ((widest + 7) / 8 * 8 + 4) << "\n";
-    // Column tile of the network products: 16 (v_mfma_f32_16x16x4f32) or 32
+    // Column tile of the fp32 network products (the split ones take 16): 16 (v_mfma_f32_16x16x4f32) or 32
     // (v_mfma_f32_32x32x2f32), as the tuning chose it; without a choice, 16 when
     // a block holds one point.  16 needs every hidden width a multiple of 16.
     // Measured on 2->128^4->1 at 729 points, epoch kernel: one point per block
@@ -714,21 +721,27 @@ static void emit_prologue(std::ostream& o, const Tables& t, const std::vector<in
         int col_tile = net_points_per_block == 1 ? 16 : 32;
         if (tuning.col_tile == 16 || tuning.col_tile == 32) col_tile = tuning.col_tile;
         if (!hidden16) col_tile = 32;
+        if (split_products(neurons)) col_tile = 16;
         o << "#define CPDE_COL_TILE " << col_tile << "\n";
     }
+    if (split_products(neurons)) o << "#define CPDE_SPLIT_PRODUCTS 1\n";
+    o << "#define CPDE_PLANE_STRIDE " << ((widest + 31) / 32 * 32 + 8) << "\n";
     const int forward_cap = forward_split_cap(t, tuning);
     o << "#define CPDE_MAX_SPLIT " << forward_cap << "\n";
     // One LDS tile instead of two when every composition has whole columns per
-    // lane (no split): a lane then reads a column's z rows and writes its y
-    // rows in place, and the products wait for every wave's operand reads
-    // before they store.  Half the LDS per workgroup.
-    if (tuning.alias && alias_tiles(t, neurons, tuning)) o << "#define CPDE_ALIAS_TILES 1\n";
+    // lane (no split): every lane takes its columns' z rows before any writes
+    // its y rows over them, and the products wait for every wave's operand
+    // reads before they store.  Two fifths less LDS per workgroup: on request,
+    // or where two tiles would pass the workgroup's 160 KB.
+    const int columns = (net_points_per_block * t.rows + 15) / 16 * 16;
+    const size_t tile_bytes = size_t(columns) * (6 * ((widest + 31) / 32 * 32 + 8) + 4 * ((widest + 7) / 8 * 8 + 4));
+    if ((tuning.alias || (split_products(neurons) && tile_bytes > 150 * 1024)) && alias_tiles(t, neurons, tuning))
+        o << "#define CPDE_ALIAS_TILES 1\n";
     o << "#define CPDE_MAX_SPLIT_ADJOINT " << tuning.max_split_adjoint << "\n";
     if (tuning.scaled) o << "#define CPDE_SCALED 1\n";
     if (tuning.inkernel_wgrad) o << "#define CPDE_INKERNEL_WGRAD 1\n";
     if (tuning.b_pairs) o << "#define CPDE_B_PAIRS 1\n";
     if (tuning.stamps) o << "#define CPDE_STAMPS 1\n";
-    if (tuning.tier_prio) o << "#define CPDE_TIER_PRIO " << tuning.tier_prio << "\n#define CPDE_TIER_CUS " << tuning.tier_cus << "\n";
     // row splits of the compositions used by the network-fused kernels (scaled
     // forward compositions split over mirror lanes instead)
     std::vector<int> splits;
@@ -746,6 +759,9 @@ static void emit_prologue(std::ostream& o, const Tables& t, const std::vector<in
     o << compose_source(t, splits, tuning.scaled != 0);
     o << kFusedSource;
 }
+
+// Template argument of a phase: whether it leaves X as a product's operand.
+static const char* operand(bool yes) { return yes ? "true" : "false"; }
 
 // Body of a one-pass epoch kernel: the forward of the workgroup's points, the
 // output values and the output adjoint of its columns kept in LDS (O), the
@@ -772,22 +788,17 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    float* const S = T;\n"
        << "#endif\n"
        << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n"
-       << "    tier_priority(a, 0);\n"
        << prefetch << "    const float xin = input_ahead<" << neurons[0] << ">(a, p0, npts);  // for the input gradient\n"
-       << "    net_input<" << neurons[0] << ", " << neurons[1] << ">(a, X, p0, npts);\n"
-       << "    zero_pad(X, " << neurons[1] << ", " << (neurons[1] + 7) / 8 * 8 << ");\n"
+       << "    net_input<" << neurons[0] << ", " << neurons[1] << ", " << operand(L > 3) << ">(a, X, p0, npts);\n"
        << "    __syncthreads();\n"
        << after_input;
     // the last hidden layer's y (read from X by the output layer's partial) and
     // the first one's dE/dz (read from X by the input transition's) stay in the
     // workgroup: no later launch reads them
-    int marker = 0;
     for (int t = 1; t + 2 < L; ++t)
-        ep << "    tier_priority(a, " << ++marker << ");\n"
-           << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << (t + 3 == L ? ", false" : "") << ">(a, " << t
-           << ", X, T, p0, npts);\n";
+        ep << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
+           << (t + 3 == L ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
     const std::string last = std::to_string(neurons[L - 2]);
-    ep << "    tier_priority(a, " << ++marker << ");\n";
     ep << "    UAhead<" << last << ", output_adjoint_split<" << last
        << ">()> ua;  // the last hidden layer's u rows, in flight during the output layer and the cost\n"
        << "    u_ahead<" << last << ", output_adjoint_split<" << last << ">()>(a, " << L - 2 << ", p0, npts, ua);\n"
@@ -795,13 +806,11 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    w_ahead<" << last << ", " << NO << ">(a, " << L - 2 << ", npts, wa);\n"
        << "    net_output<" << neurons[L - 2] << ", " << NO << ">(a, " << L - 2 << ", X, p0, npts, O);\n"
        << "    __syncthreads();  // the output values of the block's columns are in O\n"
-       << "    tier_priority(a, " << ++marker << ");\n"
-       << cost << "    net_output_backward<" << neurons[L - 2] << ", " << NO << ", true>(a, " << L - 2
+       << cost << "    net_output_backward<" << neurons[L - 2] << ", " << NO << ", " << operand(L > 3) << ", true>(a, " << L - 2
        << ", X, p0, npts, ua, O + kNNC * " << NO << ", &wa);\n";
     for (int t = L - 3; t >= 1; --t)
-        ep << "    tier_priority(a, " << ++marker << ");\n"
-           << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << (t == 1 ? ", false" : "") << ">(a, "
-           << t << ", X, T, p0, npts);\n";
+        ep << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t > 1)
+           << (t == 1 ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
     ep << "    net_input_gradient<" << neurons[0] << ", " << neurons[1] << ", true>(a, X, p0, npts, xin);\n";
     // Diagnostics (FusedTuning::stamps): a clock stamp after every phase --
     // each call above and each barrier between them -- written over the
@@ -835,24 +844,27 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
     // the one-pass epoch runs both with the matching cost between them
     std::ostringstream fwd, bwd;
     fwd << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n";
-    for (int t = 1; t + 2 < L; ++t)
-        fwd << "    net_transpose<" << neurons[t] << ", " << neurons[t + 1] << ">(a, " << t << ");\n";
-    fwd << "    net_input<" << neurons[0] << ", " << neurons[1] << ">(a, X, p0, npts);\n"
-        << "    zero_pad(X, " << neurons[1] << ", " << (neurons[1] + 7) / 8 * 8 << ");\n"
+    if (!split_products(neurons))
+        for (int t = 1; t + 2 < L; ++t)
+            fwd << "    net_transpose<" << neurons[t] << ", " << neurons[t + 1] << ">(a, " << t << ");\n";
+    fwd << "    net_input<" << neurons[0] << ", " << neurons[1] << ", " << operand(L > 3) << ">(a, X, p0, npts);\n"
         << "    __syncthreads();\n";
     for (int t = 1; t + 2 < L; ++t)
-        fwd << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ">(a, " << t << ", X, T, p0, npts);\n";
+        fwd << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L) << ">(a, " << t
+            << ", X, T, p0, npts);\n";
     fwd << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
     {
         const std::string last = std::to_string(neurons[L - 2]);
         bwd << "    UAhead<" << last << ", output_adjoint_split<" << last << ">()> ua;\n    u_ahead<" << last
             << ", output_adjoint_split<" << last << ">()>(a, " << L - 2
             << ", p0, npts, ua);\n"
-            << "    net_output_backward<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2
+            << "    net_output_backward<" << neurons[L - 2] << ", " << neurons[L - 1] << ", " << operand(L > 3) << ">(a, "
+            << L - 2
             << ", X, p0, npts, ua);\n";
     }
     for (int t = L - 3; t >= 1; --t)
-        bwd << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ">(a, " << t << ", X, T, p0, npts);\n";
+        bwd << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t > 1) << ">(a, " << t
+            << ", X, T, p0, npts);\n";
     bwd << "    net_input_gradient<" << neurons[0] << ", " << neurons[1] << ">(a, X, p0, npts);\n";
     const std::string tiles = tile_declarations();
     const std::string nt = std::to_string(tuning.net_threads);

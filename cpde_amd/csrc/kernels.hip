@@ -763,11 +763,12 @@ struct OptimizerArgs {
     float* S[kMaxTransitions];   // RPROP step / Adam first moment
     float* Ga[kMaxTransitions];  // active gradient
     float* Gi[kMaxTransitions];  // inactive gradient / Adam second moment
-    float* WT[kMaxTransitions];  // row-major copy of the weights, kept current by RPROP and Adam
+    void* WS[kMaxTransitions];  // the weights as product operands (or null), kept current by RPROP and Adam
     int NO[kMaxTransitions], NI[kMaxTransitions];
     int begin[kMaxTransitions + 1];
     int block_begin[kMaxTransitions + 1];  // blocks of kOptimizerThreads entries, per transition
     int transitions;
+    int split;  // WS: split bf16 operands, else the row-major fp32 copy
     // guarded: update only if the epoch's scalars pass the acceptance rule;
     // the first lane of the grid leaves the verdict in *verdict (if non-null)
     UpdateGuard guard;
@@ -878,10 +879,36 @@ __device__ __forceinline__ bool update_applies(const OptimizerArgs& a, bool fini
 }
 
 
-// Entry j = o + NO*i of a weight block into its row-major copy (bias column i = NI excluded).
-__device__ __forceinline__ void copy_transposed(const OptimizerArgs& a, int t, int j, float w) {
+// Weight w(o, i) of an n_in -> n_out transition into its product operands
+// (Net::ws): split exactly into three bf16 values, at 16-neuron block, 32-k step,
+// plane, lane (q, j) and place in the lane's eight -- the forward's with m = o,
+// k = i, the backward's with m = i, k = o.
+__device__ __forceinline__ void weight_operand(unsigned short* ws, int n_in, int n_out, int o, int i, float w) {
+    const float r = w - upper_half(w);
+    const unsigned mid = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r, r}, bf16x2));
+    const unsigned short plane[3] = {static_cast<unsigned short>(__float_as_uint(w) >> 16),
+                                     static_cast<unsigned short>(mid),
+                                     static_cast<unsigned short>(__float_as_uint(r - __uint_as_float(mid << 16)) >> 16)};
+    auto put = [&](unsigned short* base, int m, int k, int width) {
+        unsigned short* at = base + ((m >> 4) * ((width + 31) / 32) + (k >> 5)) * 3 * 512 +
+                             (((k >> 3) & 3) * 16 + (m & 15)) * 8 + (k & 7);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) at[p * 512] = plane[p];
+    };
+    put(ws, o, i, n_in);
+    put(ws + (n_out + 15) / 16 * ((n_in + 31) / 32) * 3 * 512, i, o, n_out);
+}
+
+__device__ __forceinline__ void product_operand(void* ws, bool split, int n_in, int n_out, int o, int i, float w) {
+    if (split) weight_operand(static_cast<unsigned short*>(ws), n_in, n_out, o, i, w);
+    else static_cast<float*>(ws)[i + n_in * o] = w;
+}
+
+// Entry j = o + NO*i of a weight block into its product operands (not the bias column i = NI).
+__device__ __forceinline__ void copy_operands(const OptimizerArgs& a, int t, int j, float w) {
+    if (!a.WS[t]) return;
     const int i = j / a.NO[t], o = j - i * a.NO[t];
-    if (i < a.NI[t]) a.WT[t][i + a.NI[t] * o] = w;
+    if (i < a.NI[t]) product_operand(a.WS[t], a.split, a.NI[t], a.NO[t], o, i, w);
 }
 
 
@@ -923,7 +950,7 @@ __device__ __forceinline__ void rprop_update(const OptimizerArgs& a, int t, int 
     a.Ga[t][j] = kept_g;
     a.W[t][j] = kept;
     a.S[t][j] = s;
-    copy_transposed(a, t, j, kept);
+    copy_operands(a, t, j, kept);
 }
 
 // grad_t[m + M*n] (+)= sum over splits of the partials of entry (m, n), n = N
@@ -1484,6 +1511,7 @@ static unsigned reduce_grid(const ReduceArgs& a) {
 void launch_reduce_rprop(Device& d, const ReduceArgs& a, Net& net, int first) {
     OptimizerArgs o{};
     o.transitions = a.transitions;
+    o.split = net.split;
     for (int k = 0; k < a.transitions; ++k) {
         const int t = first + k;
         const int act = net.active[t], inact = act == 1 ? 2 : 1;
@@ -1492,7 +1520,7 @@ void launch_reduce_rprop(Device& d, const ReduceArgs& a, Net& net, int first) {
         o.S[k] = net.state[3][t];
         o.Ga[k] = net.state[act][t];
         o.Gi[k] = net.state[inact][t];
-        o.WT[k] = net.wt[t];
+        o.WS[k] = net.ws[t];
         o.NO[k] = net.neurons[t + 1];
         o.NI[k] = net.neurons[t];
     }
@@ -2023,43 +2051,43 @@ void launch_grad_stats(Device& d, const float* const* g, const int* counts, int 
     HIP_CHECK(hipGetLastError());
 }
 
-// Row-major copies WT[i + n_in*o] = W[o + n_out*i] of several weight blocks in
-// one launch (the network-fused backward's product operands).
-struct TransposeArgs {
+// The product operands of several weight blocks in one launch.
+struct WeightOperandArgs {
     const float* W[kMaxTransitions];
-    float* WT[kMaxTransitions];
+    void* WS[kMaxTransitions];
     int n_in[kMaxTransitions], n_out[kMaxTransitions];
     int begin[kMaxTransitions + 1];
-    int transitions;
+    int transitions, split;
 };
 
-__global__ void transpose_kernel(TransposeArgs a) {
+__global__ __launch_bounds__(256) void weight_operand_kernel(WeightOperandArgs a) {
     const int total = a.begin[a.transitions];
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < total; e += blockDim.x * gridDim.x) {
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < total; e += 256 * gridDim.x) {
         int t = 0;
         while (t + 1 < a.transitions && e >= a.begin[t + 1]) ++t;
-        const int local = e - a.begin[t], ni = a.n_in[t];
-        const int o = local / ni, i = local - o * ni;
-        a.WT[t][local] = a.W[t][o + a.n_out[t] * i];
+        const int local = e - a.begin[t];
+        const int i = local / a.n_out[t], o = local - i * a.n_out[t];
+        product_operand(a.WS[t], a.split, a.n_in[t], a.n_out[t], o, i, a.W[t][local]);
     }
 }
 
-void launch_transpose(Device& d, const float* const* W, float* const* WT, const int* n_in, const int* n_out,
-                      int count) {
+void launch_weight_operands(Device& d, const float* const* W, void* const* WS, const int* n_in, const int* n_out,
+                            int count, bool split) {
     for (int first = 0; first < count; first += kMaxTransitions) {
-        TransposeArgs a{};
+        WeightOperandArgs a{};
+        a.split = split;
         a.transitions = std::min(kMaxTransitions, count - first);
         a.begin[0] = 0;
         for (int k = 0; k < a.transitions; ++k) {
             a.W[k] = W[first + k];
-            a.WT[k] = WT[first + k];
+            a.WS[k] = WS[first + k];
             a.n_in[k] = n_in[first + k];
             a.n_out[k] = n_out[first + k];
             a.begin[k + 1] = a.begin[k] + n_in[first + k] * n_out[first + k];
         }
         if (!a.begin[a.transitions]) continue;
         const int blocks = std::max(1, std::min(1024, (a.begin[a.transitions] + 255) / 256));
-        hipLaunchKernelGGL(transpose_kernel, blocks, 256, 0, d.stream, a);
+        hipLaunchKernelGGL(weight_operand_kernel, blocks, 256, 0, d.stream, a);
         HIP_CHECK(hipGetLastError());
     }
 }
@@ -2161,7 +2189,7 @@ __global__ __launch_bounds__(kOptimizerThreads) void adam_kernel(OptimizerArgs a
         const float nW = float(double(w) - double(lr * mh) / (double(sqrtf(vh)) + 1e-8));
         const float kept = fabsf(nW) <= 20.0f ? nW : w;
         a.W[t][j] = kept;
-        copy_transposed(a, t, j, kept);
+        copy_operands(a, t, j, kept);
     }
 }
 
@@ -2182,6 +2210,7 @@ static void for_transition_groups(Net& net, F launch) {
     const int T = net.layers - 1;
     for (int first = 0; first < T; first += kMaxTransitions) {
         OptimizerArgs a{};
+        a.split = net.split;
         a.transitions = std::min(kMaxTransitions, T - first);
         a.begin[0] = 0;
         a.block_begin[0] = 0;
@@ -2192,7 +2221,7 @@ static void for_transition_groups(Net& net, F launch) {
             a.S[k] = net.state[3][t];
             a.Ga[k] = net.state[act][t];
             a.Gi[k] = net.state[inact][t];
-            a.WT[k] = net.wt[t];
+            a.WS[k] = net.ws[t];
             a.NO[k] = net.neurons[t + 1];
             a.NI[k] = net.neurons[t];
             a.begin[k + 1] = a.begin[k] + net.param_count(t);
@@ -2245,7 +2274,7 @@ void launch_rprop(Device& d, Net& net, const UpdateGuard* guard, const ScalarPub
     });
     if (guard) return;  // the caller switches the buffers once it knows whether the update applied
     for (auto& act : net.active) act = act == 1 ? 2 : 1;
-    net.wt_current = true;
+    net.ws_current = true;
 }
 
 void launch_adam(Device& d, Net& net, int step, float lr, const UpdateGuard* guard, const ScalarPublish* publish,
@@ -2264,7 +2293,7 @@ void launch_adam(Device& d, Net& net, int step, float lr, const UpdateGuard* gua
         hipLaunchKernelGGL(adam_kernel, blocks, kOptimizerThreads, 0, d.stream, a, lr, b1, b2, b1t, b2t);
         HIP_CHECK(hipGetLastError());
     });
-    net.wt_current = true;
+    net.ws_current = true;
 }
 
 void launch_set_steps(Device& d, Net& net, float value) {
