@@ -305,6 +305,9 @@ struct NetArgsHost {
     int block_offset, block_count;  // the pass's workgroups in the launch (count 0: the whole grid)
 };
 
+// Whether a grid's workgroups are all on the device at once (four per CU).
+static bool resident(int blocks, int compute_units) { return blocks <= 4 * compute_units; }
+
 // Tuning of the fused kernels for a schema of `rows` derivative rows over chunks
 // of `width` points (0: unknown) on `compute_units` CUs, for a network of
 // `neurons`.  The network-fused kernels put as many points in a workgroup as
@@ -380,10 +383,12 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // none: order 5 (21 rows) 0.0936 / 0.0904, order 6 (28 rows) 0.1036 /
     // 0.0992; orders 1-4, several points per workgroup, within 0.3 %).
     const bool whole = rows > 32 || (rows > 16 && t.net_points_per_block == 1);
-    // (Where whole compositions leave three lanes of four idle the mirror split
-    // still pays: 2->32^2->1 at order 6 over 40 points 21.2 -> 20.7 us.)
+    // (Where whole compositions leave three lanes of four idle, and CUs without a
+    // second workgroup, the mirror split still pays: 2->32^2->1 at order 6 over 40
+    // points 21.2 -> 20.7 us; 2->48^3->1 over 8,000 240 -> 250.)
     const int widest = *std::max_element(neurons.begin(), neurons.end());
-    const bool sparse = rows > 16 && 4 * t.net_points_per_block * widest <= t.net_threads;
+    const bool sparse = rows > 16 && 4 * t.net_points_per_block * widest <= t.net_threads && width > 0 &&
+                        (width + t.net_points_per_block - 1) / t.net_points_per_block <= compute_units;
     t.max_split = std::max(1, env_int("CPDE_NET_SPLIT", whole && !sparse ? 1 : t.max_split));
     t.max_split_adjoint = std::max(1, env_int("CPDE_NET_SPLIT_ADJOINT", t.max_split_adjoint));
     t.forward_blocks = std::max(1, env_int("CPDE_NET_FWD_OCC", t.forward_blocks));
@@ -424,9 +429,16 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
 static std::shared_ptr<FusedModule> load_fused(Device& d, const Tables& t, const std::vector<int>& neurons,
                                                int width) {
     const FusedTuning tune = tuning(t.rows, width, d.compute_units, neurons);
-    const std::string src = fused_source(t, neurons, tune);
+    // the module by what its source is made from: a plan like an earlier one
+    // does not generate the text again
+    static_assert(std::is_trivially_copyable<FusedTuning>::value, "tuning is part of the module's key");
+    std::string key;
+    for (const std::vector<int>* part : {&t.table, &neurons})
+        key.append(reinterpret_cast<const char*>(part->data()), part->size() * sizeof(int)) += '|';
+    key.append(std::to_string(t.rows) + "|").append(reinterpret_cast<const char*>(&tune), sizeof tune);
     for (auto& kv : d.fused_modules)
-        if (kv.first == src) return kv.second;
+        if (kv.first == key) return kv.second;
+    const std::string src = fused_source(t, neurons, tune);
     std::string log;
     const std::vector<char> code = compile_module(src, device_arch(d.ordinal), &log);
     auto m = std::make_shared<FusedModule>();
@@ -449,7 +461,7 @@ static std::shared_ptr<FusedModule> load_fused(Device& d, const Tables& t, const
         HIP_CHECK(
             hipModuleGetFunction(&m->hidden_backward[k], m->module, ("hidden_backward_" + std::to_string(k)).c_str()));
     }
-    d.fused_modules.emplace_back(src, m);
+    d.fused_modules.emplace_back(key, m);
     return m;
 }
 
@@ -967,7 +979,23 @@ static int epoch_blocks(const Plan& p) {
 // grids keep separate launches, where the forward has its own, higher occupancy.
 // CPDE_ONE_PASS=0 forces the separate launches (same kernels otherwise).
 static bool one_pass_fits(const Plan& p) {
-    return env_int("CPDE_ONE_PASS", 1) && p.fused && p.network && epoch_blocks(p) <= 4 * p.net->dev->compute_units;
+    return env_int("CPDE_ONE_PASS", 1) && p.fused && p.network && resident(epoch_blocks(p), p.net->dev->compute_units);
+}
+
+// Whether a matching epoch runs in one pass: also over longer grids, where no
+// hidden layer is wider than 64 (and nobody holds a stack that it leaves
+// unwritten).  Workgroups that narrow stay many per CU with the backward's
+// registers too, so the forward alone gains nothing, and the kernel saves the
+// cost launch, two stacks and u's way through memory.  Epochs, separate -> one
+// pass: 2->50^3->1 at order 3 over 5,003 points 81 -> 72 us, 2->64^3->1 at order 2
+// over 16,384 131 -> 120, at order 0 over 200,000 377 -> 262, 2->48^3->1 at order 6
+// over 8,000 250 -> 224; wider: 2->96^3->1 at order 4 over 20,000 616 -> 633,
+// 2->256^3->1 at order 2 over 30,000 1,594 -> 1,663.
+static bool matching_one_pass(const Plan& p) {
+    if (one_pass_fits(p)) return true;
+    if (!env_int("CPDE_ONE_PASS", 1) || !p.fused || !p.network || p.net->stacks_out) return false;
+    const std::vector<int>& n = p.net->neurons;
+    return *std::max_element(n.begin() + 1, n.end() - 1) <= 64;
 }
 
 // The per-workgroup cost records of a one-pass epoch.
@@ -1641,6 +1669,7 @@ int cpde_plan_stack(cpde_plan* plan, int layer, int kind, float** device_ptr) {
         require(!(kind == 3 && !keeps_u), "u is kept only by network-fused plans for sigmoid layers");
         float* p = kind == 0 || kind == 3 ? (layer == 0 ? plan->input : n.z[layer]) : kind == 1 ? n.y[layer] : n.g[layer];
         require(p != nullptr, "stack not present for this layer");
+        if (kind == 1 || kind == 2) n.stacks_out = true;
         *device_ptr = p;
     });
 }
@@ -1748,7 +1777,7 @@ int cpde_epoch_matching(cpde_plan* plan, const float* target, int target_width, 
         require(cost_index >= 0 && cost_index < d.cost_capacity, "cost slot out of range");
         require(plan->backward, "plan has no adjoint storage");
         require(valid >= 0 && valid <= plan->width && offset >= 0, "invalid chunk range");
-        if (!one_pass_fits(*plan)) {
+        if (!matching_one_pass(*plan)) {
             if (int code = cpde_forward(plan)) throw_code(code);
             if (int code = cpde_cost_matching(plan, target, target_width, target_rows, weights, weight_samples, offset,
                                               valid, cost_index, collect, 1))
@@ -1772,7 +1801,7 @@ int cpde_epoch_matching_rprop(cpde_plan* plan, const float* target, int target_w
         require(cost_index >= 0 && cost_index < d.cost_capacity, "cost slot out of range");
         require(plan->backward, "plan has no adjoint storage");
         require(valid >= 0 && valid <= plan->width && offset >= 0, "invalid chunk range");
-        if (!one_pass_fits(*plan) || n.layers - 1 > kMaxTransitions) {
+        if (!matching_one_pass(*plan) || n.layers - 1 > kMaxTransitions) {
             if (int code = cpde_epoch_matching(plan, target, target_width, target_rows, weights, weight_samples, offset,
                                                valid, cost_index, collect, accumulate))
                 throw_code(code);

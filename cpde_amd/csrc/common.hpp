@@ -120,6 +120,10 @@ struct Net {
     std::vector<float*> z, y, g;      // per layer
     std::vector<size_t> capacity;     // floats per layer buffer
     uint64_t generation = 0;
+    // a caller holds a stack's pointer (cpde_plan_stack): epochs over more
+    // workgroups than fit on the device together stay separate launches, which
+    // write every stack
+    bool stacks_out = false;
     // split-K partial buffer for the weight-gradient contraction
     float* partials = nullptr;
     size_t partial_capacity = 0;
@@ -300,7 +304,7 @@ struct Device {
     double trace_ms[kTraceKinds] = {}, trace_work[kTraceKinds] = {};
     uint64_t trace_launches[kTraceKinds] = {};
     void fold_trace();
-    // fused modules compiled on this device, by source text
+    // fused modules compiled on this device (by schema, network and tuning), and the others by source text
     std::vector<std::pair<std::string, std::shared_ptr<FusedModule>>> fused_modules;
     std::vector<std::pair<std::string, std::shared_ptr<RowsModule>>> rows_modules;
     std::vector<std::pair<std::string, std::shared_ptr<ExpressionEpoch>>> expression_epochs;

@@ -768,7 +768,7 @@ static const char* operand(bool yes) { return yes ? "true" : "false"; }
 // cost stage `cost` between them (it fills O's second half), then the
 // backward.  The row-major weight copies are written before the launch.
 static std::string epoch_body(const std::vector<int>& neurons, const std::string& prefetch, const std::string& cost,
-                              bool stamps, const std::string& after_input = "") {
+                              const FusedTuning& tuning, const std::string& after_input = "") {
     const int L = int(neurons.size()), NO = neurons[L - 1];
     std::ostringstream ep;
     // S: the cost stage's scratch (matching terms, or a double and an int per
@@ -815,7 +815,7 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
     // Diagnostics (FusedTuning::stamps): a clock stamp after every phase --
     // each call above and each barrier between them -- written over the
     // block's output stack when the epoch ends.
-    if (!stamps) return ep.str();
+    if (!tuning.stamps) return ep.str();
     std::istringstream lines(ep.str());
     std::ostringstream st;
     std::string line;
@@ -884,7 +884,7 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
                                  ", S, p0, npts, O, O + kNNC * " + std::to_string(NO) + ", pre);\n";
         o << "extern \"C\" __global__ __launch_bounds__(" << nt << ", " << tuning.backward_blocks
           << ") void network_epoch_k(NetArgs a, MatchArgs m, int points) {\n"
-          << epoch_body(neurons, prefetch, cost, tuning.stamps != 0, after_input) << "}\n";
+          << epoch_body(neurons, prefetch, cost, tuning, after_input) << "}\n";
     }
     o << "\nextern \"C\" __global__ __launch_bounds__(256) void input_layer_k(const float* W, const float* X, float* Z,"
          " float* Y, int points) { input_layer<"
@@ -924,7 +924,7 @@ std::string expression_epoch_source(const Tables& t, const std::vector<int>& neu
     emit_prologue(o, t, neurons, tuning);
     o << "extern \"C\" __global__ __launch_bounds__(" << tuning.net_threads << ", " << tuning.backward_blocks
       << ") void network_epoch_expression_k(NetArgs a, ExpressionArgs e, int points) {\n"
-      << epoch_body(neurons, expression_ahead_line(), expression_cost(L, NO), tuning.stamps != 0) << "}\n";
+      << epoch_body(neurons, expression_ahead_line(), expression_cost(L, NO), tuning) << "}\n";
     return o.str();
 }
 
@@ -951,7 +951,7 @@ std::string expression_pair_source(const Tables& t0, const FusedTuning& u0, cons
              << (leaf ? program1 : program0) << "\n#undef expression\n#define CPDE_EXPRESSION_EPOCH 1\n";
         emit_prologue(part, leaf ? t1 : t0, neurons, leaf ? u1 : u0);
         part << "__device__ __forceinline__ void epoch(const NetArgs& a, const ExpressionArgs& e, int points) {\n"
-             << epoch_body(neurons, expression_ahead_line(), cost, (leaf ? u1 : u0).stamps != 0) << "}\n";
+             << epoch_body(neurons, expression_ahead_line(), cost, leaf ? u1 : u0) << "}\n";
         const std::string text = part.str();
         o << "namespace cpde_leaf" << leaf << " {\n" << text << "}  // namespace cpde_leaf" << leaf << "\n";
         std::istringstream lines(text);

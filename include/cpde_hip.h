@@ -190,12 +190,14 @@ int cpde_cost_matching(cpde_plan* plan, const float* target, int target_width, c
  * (cuda/cpde_server.cu:223-257): cpde_forward, cpde_cost_matching(gradient=1)
  * and cpde_backward(accumulate) with the same arguments.  The reference runs
  * them as separate launches; on the network-fused kernels, when the chunk's
- * workgroups fit on the device together, this is one launch (a point's
- * matching terms depend on that point alone), the cost's finish and the
- * weight-gradient contraction.  The input chunk must be activated.  That one
- * launch leaves two stacks unwritten, which no later launch reads: y of the
- * last hidden layer and dE/dz of the first (cpde_plan_stack kinds 1 and 2);
- * read them after the separate calls instead. */
+ * workgroups fit on the device together or no hidden layer is wider than 64,
+ * this is one launch (a point's matching terms depend on that point alone), the
+ * cost's finish and the weight-gradient contraction.  The input chunk must be
+ * activated.  That one launch leaves two stacks unwritten, which no later
+ * launch reads: y of the last hidden layer and dE/dz of the first
+ * (cpde_plan_stack kinds 1 and 2); read them after the separate calls instead.
+ * (Chunks of more workgroups than fit together run as the separate calls, and
+ * write them, once a stack's pointer has been asked for on the network.) */
 int cpde_epoch_matching(cpde_plan* plan, const float* target, int target_width, const int* target_rows,
                         const float* weights, int weight_samples, int offset, int valid, int cost_index, int collect,
                         int accumulate);

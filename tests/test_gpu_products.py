@@ -48,6 +48,34 @@ def test_split_products(device, variables, order, neurons, points, chunk):
         assert rel_l2(g, w) < 1e-4, t
 
 
+@pytest.mark.parametrize('variables,order,neurons,points,chunk', [
+    (2, 5, [2, 64, 40, 1], 1031, 0),     # 21 rows: one point per workgroup, a few past the resident grid
+    (1, 3, [1, 33, 64, 64, 1], 8301, 8250),  # four rows: several points, a ragged second chunk
+    (2, 0, [2, 20, 1], 33001, 0),        # one hidden layer, one row
+])
+def test_long_one_pass_of_narrow_layers(device, variables, order, neurons, points, chunk):
+    """One-pass epochs over more workgroups than fit on the device together:
+    loss and gradients of separate launches; and once a stack's pointer is out,
+    every stack as separate launches leave it."""
+    wl = workload(variables, order, neurons, points, chunk, seed=37)
+    print(f'[case] long one pass neurons={neurons} rows={wl.rows} points={points}', flush=True)
+    got = []
+    for one_pass in (True, False):
+        run = hip.MatchingRun(device, wl, one_pass=one_pass)
+        run.step()
+        device.synchronize()
+        got.append((run.loss(), run.gradients()))
+        run.plan.stack_ptr(1, 1)
+        run.step()
+        device.synchronize()
+        last = points % (chunk or points) or points   # points of the chunk the stacks hold
+        got[-1] += ([run.plan.stack(layer, kind)[:last] for layer in range(1, len(neurons) - 1) for kind in (1, 2, 3)],)
+        run.close()
+    assert abs(got[0][0] / got[1][0] - 1) < 1e-12
+    for a, b in zip(got[0][1] + got[0][2], got[1][1] + got[1][2]):
+        assert np.array_equal(a, b)
+
+
 def test_forward_sees_weights_written_through_a_held_pointer(device):
     """A program that keeps a weights pointer and writes through it again: each
     separate forward runs on what it wrote, on split operands too."""
