@@ -449,6 +449,7 @@ static std::shared_ptr<FusedModule> load_fused(Device& d, const Tables& t, const
     m->inkernel_wgrad = tune.inkernel_wgrad != 0;
     HIP_CHECK(hipModuleLoadData(&m->module, code.data()));
     HIP_CHECK(hipModuleGetFunction(&m->network_forward, m->module, "network_forward_k"));
+    HIP_CHECK(hipModuleGetFunction(&m->network_values, m->module, "network_values_k"));
     HIP_CHECK(hipModuleGetFunction(&m->network_backward, m->module, "network_backward_k"));
     HIP_CHECK(hipModuleGetFunction(&m->network_epoch, m->module, "network_epoch_k"));
     HIP_CHECK(hipModuleGetFunction(&m->input_layer, m->module, "input_layer_k"));
@@ -567,9 +568,15 @@ static void fused_forward(Plan& p) {
         double flops = 0;
         for (int t = 0; t + 1 < L; ++t) flops += 2.0 * n.neurons[t] * n.neurons[t + 1] * cols;
         TraceScope trace(d, kTraceNetworkForward, flops);
-        launch_module(d, fm.network_forward, unsigned((width + fm.net_points_per_block - 1) / fm.net_points_per_block),
-                      1, args, unsigned(fm.net_threads));
-        n.ws_current = true;  // fp32 products: written by the forward's side job
+        // A plan without a backward writes its outputs alone: nothing reads the
+        // layers' stacks, which are most of such a forward's bytes (65,536 points
+        // 2->128^4->1 83 -> 54 us; 10 rows of 32,768 points 3->128^5->1 470 -> 293).
+        const bool values = !p.backward && !n.stacks_out && !n.bound;
+        launch_module(d, values ? fm.network_values : fm.network_forward,
+                      unsigned((width + fm.net_points_per_block - 1) / fm.net_points_per_block), 1, args,
+                      unsigned(fm.net_threads));
+        n.values_only = values ? &p : nullptr;
+        if (!values) n.ws_current = true;  // fp32 products: written by the forward's side job
         return;
     }
     {
@@ -1189,6 +1196,7 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
     int width = p.width;
     const double cols = double(p.columns());
     const int blocks = epoch_blocks(p);
+    n.values_only = nullptr;
     // a held epoch this one cannot join goes out before anything of this one
     if (d.held && d.held->open && (!program || !epoch_pairs() || d.held->plan == &p || d.held->plan->net != &n))
         flush_held(d);
@@ -1580,6 +1588,7 @@ int cpde_plan_destroy(cpde_plan* plan) {
         if (!plan) return;
         Net& n = *plan->net;
         sync_stream(*n.dev, __LINE__);
+        if (n.values_only == plan) n.values_only = nullptr;
         if (n.bound && n.bound->plan == plan) {
             swap_binding(n, *plan, *n.bound);
             n.bound = nullptr;
@@ -1669,7 +1678,10 @@ int cpde_plan_stack(cpde_plan* plan, int layer, int kind, float** device_ptr) {
         require(!(kind == 3 && !keeps_u), "u is kept only by network-fused plans for sigmoid layers");
         float* p = kind == 0 || kind == 3 ? (layer == 0 ? plan->input : n.z[layer]) : kind == 1 ? n.y[layer] : n.g[layer];
         require(p != nullptr, "stack not present for this layer");
-        if (kind == 1 || kind == 2) n.stacks_out = true;
+        if (layer > 0 && layer + 1 < n.layers) {
+            n.stacks_out = true;
+            if (n.values_only == plan && !n.dev->capturing) fused_forward(*plan);  // the stacks it left out
+        }
         *device_ptr = p;
     });
 }
@@ -1698,6 +1710,7 @@ int cpde_activate(cpde_plan* plan, const float* data, int data_width, const int*
         require(valid >= 0 && valid <= plan->width && offset >= 0 && offset + valid <= data_width,
                 "invalid chunk range");
         reserve_arena(n, *plan);
+        if (n.values_only == plan) n.values_only = nullptr;  // its input is another now
         launch_activate(d, plan->input, data, data_width, n.neurons[0], plan_rows(*plan, rows), plan->rows, plan->width,
                         offset, valid);
     });
@@ -1712,6 +1725,7 @@ int cpde_forward(cpde_plan* plan) {
             fused_forward(*plan);
             return;
         }
+        n.values_only = nullptr;
         const int cols = int(plan->columns());
         for (int t = 0; t + 1 < n.layers; ++t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];

@@ -120,10 +120,12 @@ struct Net {
     std::vector<float*> z, y, g;      // per layer
     std::vector<size_t> capacity;     // floats per layer buffer
     uint64_t generation = 0;
-    // a caller holds a stack's pointer (cpde_plan_stack): epochs over more
-    // workgroups than fit on the device together stay separate launches, which
-    // write every stack
+    // a caller holds a stack's pointer (cpde_plan_stack): from then on forwards
+    // without a backward write every stack, and epochs over more workgroups than
+    // fit on the device together stay separate launches, which do
     bool stacks_out = false;
+    // the plan whose forward ran last on the arena, where it wrote no stacks
+    const struct Plan* values_only = nullptr;
     // split-K partial buffer for the weight-gradient contraction
     float* partials = nullptr;
     size_t partial_capacity = 0;
@@ -374,7 +376,7 @@ struct FusedModule {
     hipModule_t module = nullptr;
     hipFunction_t input_layer = nullptr, output_backward = nullptr;
     std::vector<hipFunction_t> hidden_forward, hidden_backward;  // per transition (index t)
-    hipFunction_t network_forward = nullptr, network_backward = nullptr, network_epoch = nullptr;
+    hipFunction_t network_forward = nullptr, network_values = nullptr, network_backward = nullptr, network_epoch = nullptr;
     int points_per_block = 2, net_points_per_block = 1, net_threads = 256;
     bool scaled = false;  // sigmoid stacks of the network kernels hold row alpha / alpha! (dE/dz: times alpha!)
     bool inkernel_wgrad = false;  // the network backward writes every hidden transition's per-block partial

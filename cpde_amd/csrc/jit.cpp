@@ -853,6 +853,15 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
         fwd << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L) << ">(a, " << t
             << ", X, T, p0, npts);\n";
     fwd << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
+    // the forward of a plan without a backward: outputs alone, no layer's stacks
+    std::ostringstream val;
+    val << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n"
+        << "    net_input<" << neurons[0] << ", " << neurons[1] << ", " << operand(L > 3) << ", false>(a, X, p0, npts);\n"
+        << "    __syncthreads();\n";
+    for (int t = 1; t + 2 < L; ++t)
+        val << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
+            << ", false, false>(a, " << t << ", X, T, p0, npts);\n";
+    val << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
     {
         const std::string last = std::to_string(neurons[L - 2]);
         bwd << "    UAhead<" << last << ", output_adjoint_split<" << last << ">()> ua;\n    u_ahead<" << last
@@ -871,6 +880,9 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
     o << "\nextern \"C\" __global__ __launch_bounds__(" << nt << ", " << tuning.forward_blocks
       << ") void network_forward_k(NetArgs a, int points) {\n"
       << tiles << fwd.str() << "}\n";
+    o << "extern \"C\" __global__ __launch_bounds__(" << nt << ", " << tuning.forward_blocks
+      << ") void network_values_k(NetArgs a, int points) {\n"
+      << tiles << val.str() << "}\n";
     o << "extern \"C\" __global__ __launch_bounds__(" << nt << ", " << tuning.backward_blocks
       << ") void network_backward_k(NetArgs a, int points) {\n"
       << tiles << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n" << bwd.str() << "}\n";

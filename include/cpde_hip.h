@@ -159,7 +159,10 @@ int cpde_stacks_destroy(cpde_stacks* stacks);
  * selecting the data row of plan row r; lanes [valid, width) are zeroed. */
 int cpde_activate(cpde_plan* plan, const float* data, int data_width, const int* rows, int offset, int valid);
 /* network::feedforward (cuda/cpde_engine.cuh:889-913): every layer's linear step
- * (fp32 MFMA, bias on the value row) and sigmoid composition through order 6. */
+ * (fp32 accuracy on MFMA, bias on the value row) and sigmoid composition through
+ * order 6.  A plan without a backward writes its output stack alone on the
+ * network-fused kernels; the layers' stacks follow when cpde_plan_stack first
+ * asks for one, and with every forward from then on. */
 int cpde_forward(cpde_plan* plan);
 /* Copy the output stack's valid lanes to wire layout dest [dest_rows][dest_width][n_out]
  * (device), plan row r going to dest row rows[r] (Server::evaluate :171-183). */
