@@ -396,6 +396,102 @@ __device__ __forceinline__ void wgrad_thin(const WgradArgs& a, int t, int split,
     }
 }
 
+// wgrad_thin where the narrow side is at most 4 and the wide side a multiple of
+// 4: a lane takes four adjacent wide entries of every S-th column, so that a
+// column is one run of float4 loads, eight columns in flight.  The scalar form
+// waits on a round of loads per four columns and a 64-entry lane range.
+constexpr int kThinNarrow = 4;
+__device__ __forceinline__ void wgrad_thin4(const WgradArgs& a, int t, int split, float* red) {
+    const int M = a.M[t], N = a.N[t], K = a.K[t], R = a.R[t];
+    const int kbegin = split * a.kchunk[t], kend = min(K, kbegin + a.kchunk[t]);
+    const bool wide_m = M >= N;  // otherwise the wide side is n
+    const int wide = wide_m ? M : N, narrow = wide_m ? N : M;  // wide: at least 4
+    const float* __restrict__ wp = wide_m ? a.G[t] : a.Y[t];
+    const float* __restrict__ np = wide_m ? a.Y[t] : a.G[t];
+    float* P = a.partial[t] + size_t(split) * M * (N + 1);
+    constexpr int U = 8, Q = kThinNarrow;
+    const int lanes = min(wide / 4, 256), S = 256 / lanes;
+    const int s = threadIdx.x / lanes, w = threadIdx.x - s * lanes;
+    const int rstep = S % R;
+    for (int w0 = 0; w0 < wide; w0 += 4 * lanes) {
+        const int wi = w0 + 4 * w;
+        floatx4 acc[Q], ones = {0.0f, 0.0f, 0.0f, 0.0f};  // ones: the wide side's sum over value rows
+        float bias[Q];                                    // and the narrow side's
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            acc[q] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            bias[q] = 0.0f;
+        }
+        if (s < S && wi < wide) {
+            int row = (kbegin + s) % R;  // the column's row of its point
+            for (int k = kbegin + s; k < kend; k += U * S) {
+                floatx4 wv[U];
+                float nv[U][Q];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {  // past the end: the last column again, not added
+                    const size_t kk = size_t(min(k + u * S, kend - 1));
+                    wv[u] = *reinterpret_cast<const floatx4*>(wp + kk * wide + wi);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) nv[u][q] = q < narrow ? np[kk * narrow + q] : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (k + u * S < kend) {
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) acc[q] += wv[u] * nv[u][q];
+                        if (row == 0) {
+                            ones += wv[u];
+#pragma unroll
+                            for (int q = 0; q < Q; ++q) bias[q] += nv[u][q];
+                        }
+                    }
+                    row += rstep;
+                    if (row >= R) row -= R;
+                }
+            }
+        }
+        // the S streams meet in LDS in order: Q + 1 sums of four entries per lane
+        __syncthreads();
+        floatx4* const slots = reinterpret_cast<floatx4*>(red);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) slots[q * 256 + threadIdx.x] = acc[q];
+        slots[Q * 256 + threadIdx.x] = ones;
+        __syncthreads();
+        if (s == 0 && wi < wide) {
+#pragma unroll
+            for (int q = 0; q <= Q; ++q) {
+                floatx4 sum = slots[q * 256 + w];
+                for (int x = 1; x < S; ++x) sum += slots[q * 256 + x * lanes + w];
+                if (wide_m ? q < narrow || q == Q : q < narrow)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (wide_m) P[size_t(wi + i) * (N + 1) + (q == Q ? N : q)] = sum[i];
+                        else P[size_t(q) * (N + 1) + wi + i] = sum[i];
+                    }
+            }
+        }
+        if (!wide_m && w0 == 0) {
+            __syncthreads();
+            if (w == 0 && s < S)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) red[s * Q + q] = bias[q];
+            __syncthreads();
+            if (int(threadIdx.x) < M) {
+                float b = 0.0f;
+                for (int x = 0; x < S; ++x) b += red[x * Q + threadIdx.x];
+                P[size_t(threadIdx.x) * (N + 1) + N] = b;
+            }
+        }
+    }
+}
+
+// A thin transition's split.
+__device__ __forceinline__ void wgrad_thin_any(const WgradArgs& a, int t, int split, float* red) {
+    const int wide = max(a.M[t], a.N[t]), narrow = min(a.M[t], a.N[t]);
+    if (narrow <= kThinNarrow && wide % 4 == 0) wgrad_thin4(a, t, split, red);
+    else wgrad_thin(a, t, split, red);
+}
+
 // Workgroups go to the eight XCDs round-robin (workgroup b on XCD b % 8), each
 // XCD with its own L2.  This renumbering gives every XCD a contiguous range of
 // work items, so that the tiles of one split, which read the same rows of G
@@ -671,11 +767,11 @@ __device__ __forceinline__ void split_accumulate(SplitBlock<NB>& c, SA& sa, SB& 
 // 512 over 12,288 columns: 52 us, against 114 us of the fp32 instruction
 // (32 x 32 x 2, 16-column steps, scalar LDS traffic); 64 x 64 over 168,000
 // columns (M up to 64) 62 -> 22 to 29 us.
-template <bool A_K, bool VEC, int WM>
+template <bool A_K, bool VEC, int WM, int NB>
 __global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
                                                             const float* __restrict__ B, int ldb, float* __restrict__ C,
                                                             int ldc, const float* __restrict__ bias, int period) {
-    constexpr int WN = 4 / WM, TM = 64 * WM, TN = 64 * WN;
+    constexpr int WN = 4 / WM, TM = 64 * WM, TN = 16 * NB * WN;
     __shared__ __attribute__((aligned(16))) unsigned char lds[sp_lds_bytes(TM + TN)];
     unsigned char* const la = lds;
     unsigned char* const lb = lds + sp_lds_bytes(TM);
@@ -685,13 +781,13 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K,
     const int m0 = (block % tiles_m) * TM, n0 = (block / tiles_m) * TN;
     SplitStage<TM, A_K, VEC> sa(A, lda, M, m0, tid);
     SplitStage<TN, true, VEC> sb(B, ldb, N, n0, tid);
-    SplitBlock<4> c;
-    split_accumulate(c, sa, sb, 0, K, la, lb, 64 * (wave % WM), 64 * (wave / WM));
+    SplitBlock<NB> c;
+    split_accumulate(c, sa, sb, 0, K, la, lb, 64 * (wave % WM), 16 * NB * (wave / WM));
     const int q = lane >> 4, j = lane & 15;
-    const int mw = m0 + 64 * (wave % WM) + 4 * q, nw = n0 + 64 * (wave / WM) + j;
+    const int mw = m0 + 64 * (wave % WM) + 4 * q, nw = n0 + 16 * NB * (wave / WM) + j;
     const bool quads = (M | ldc) % 4 == 0 && ((reinterpret_cast<size_t>(C) | reinterpret_cast<size_t>(bias)) & 15) == 0;
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
+    for (int y = 0; y < NB; ++y) {
         const int n = nw + 16 * y;
         if (n >= N) break;
         const bool add = bias != nullptr && n % period == 0;
@@ -712,16 +808,27 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(int M, int N, int K,
     }
 }
 
+template <bool A_K, bool VEC, int WM, int NB>
+static void split_gemm_tiles(Device& d, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+                             int ldc, const float* bias, int period) {
+    constexpr int TM = 64 * WM, TN = 16 * NB * (4 / WM);
+    hipLaunchKernelGGL((split_gemm_kernel<A_K, VEC, WM, NB>), (M + TM - 1) / TM * ((N + TN - 1) / TN), 256, 0, d.stream,
+                       M, N, K, A, lda, B, ldb, C, ldc, bias, period);
+    HIP_CHECK(hipGetLastError());
+}
+
 template <bool A_K, bool VEC>
 static void split_gemm(Device& d, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
                        int ldc, const float* bias, int period) {
-    if (M <= 64)
-        hipLaunchKernelGGL((split_gemm_kernel<A_K, VEC, 1>), (N + 255) / 256, 256, 0, d.stream, M, N, K, A, lda, B, ldb,
-                           C, ldc, bias, period);
-    else
-        hipLaunchKernelGGL((split_gemm_kernel<A_K, VEC, 2>), (M + 127) / 128 * ((N + 127) / 128), 256, 0, d.stream, M,
-                           N, K, A, lda, B, ldb, C, ldc, bias, period);
-    HIP_CHECK(hipGetLastError());
+    const bool low = M <= 64;
+    const double tiles = double((M + (low ? 63 : 127)) / (low ? 64 : 128)) * ((N + (low ? 255 : 127)) / (low ? 256 : 128));
+    // Half tiles (three workgroups per CU) where the whole ones are few, so that
+    // no CU runs two beside others' one: 512 x 512 over 12,288 columns, 384 tiles,
+    // 52 -> 49 us.
+    const bool half = tiles < 4.0 * d.compute_units;
+    const auto run = low ? (half ? split_gemm_tiles<A_K, VEC, 1, 2> : split_gemm_tiles<A_K, VEC, 1, 4>)
+                         : (half ? split_gemm_tiles<A_K, VEC, 2, 2> : split_gemm_tiles<A_K, VEC, 2, 4>);
+    run(d, M, N, K, A, lda, B, ldb, C, ldc, bias, period);
 }
 
 void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_k, const float* B, int ldb, float* C,
@@ -740,11 +847,11 @@ void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a
 // overlap the other's MFMAs.
 __global__ __launch_bounds__(256, 2) void wgrad_grouped_kernel(WgradArgs a) {
     __shared__ __attribute__((aligned(16))) float lds[kWgLds];
-    static_assert(256 * 17 <= kWgLds, "thin-transition scratch exceeds the shared LDS");
+    static_assert(256 * 4 * (kThinNarrow + 1) <= kWgLds && 256 * 17 <= kWgLds, "thin-transition scratch exceeds the shared LDS");
     const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
     const int t = group_of(a.block_begin, a.transitions, b);
     const int local = b - a.block_begin[t];
-    if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin(a, t, local, lds);
+    if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin_any(a, t, local, lds);
     else if (a.tile[t] == 64) wgrad_tile<64>(a, t, local, lds);
     else wgrad_tile<128>(a, t, local, lds);
 }
@@ -1415,11 +1522,11 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, int t, int 
 #endif
 __global__ __launch_bounds__(256, CPDE_WD_MIN_BLOCKS) void wgrad_direct_kernel(WgradArgs a) {
     __shared__ __attribute__((aligned(16))) float lds[kWdLds];
-    static_assert(256 * 17 <= kWdLds, "thin-transition scratch exceeds the shared LDS");
+    static_assert(256 * 4 * (kThinNarrow + 1) <= kWdLds && 256 * 17 <= kWdLds, "thin-transition scratch exceeds the shared LDS");
     const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
     const int t = group_of(a.block_begin, a.transitions, b);
     const int local = b - a.block_begin[t];
-    if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin(a, t, local, lds);
+    if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin_any(a, t, local, lds);
     else if (a.M[t] % 4 == 0 && a.N[t] % 4 == 0) wgrad_direct_tile<true>(a, t, local, lds);
     else wgrad_direct_tile<false>(a, t, local, lds);
 }
@@ -1437,7 +1544,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_split_kernel(WgradArgs a) {
     if (a.tile[t] == 128) {
         if (vec) wgrad_split_tile<128, true>(a, t, local, lds);
         else wgrad_split_tile<128, false>(a, t, local, lds);
-    } else if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin(a, t, local, floats);
+    } else if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin_any(a, t, local, floats);
     else if (vec) wgrad_direct_tile<true>(a, t, local, floats);
     else wgrad_direct_tile<false>(a, t, local, floats);
 }
