@@ -402,6 +402,11 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // 0.0879 / 0.0876, 3->128^5->1 order 4 at 32768 points 5.20 / 5.37.
     t.b_pairs = env_int("CPDE_NET_BPAIR", t.b_pairs);
     t.scaled = env_int("CPDE_SCALED", t.scaled) ? 1 : 0;
+    // Wave priorities by dispatch round (tier_raise in the generated source).
+    const int blocks = (width + t.net_points_per_block - 1) / t.net_points_per_block;
+    if (env_int("CPDE_NET_TIERS", 1) && !split_products(neurons) && blocks > compute_units &&
+        resident(blocks, compute_units))
+        t.tier_cus = compute_units;
     // Diagnostics: clock stamps of the one-pass epoch's phases, written over
     // the output stack (cpde_amd/stamps.py reads them back).
     t.stamps = env_int("CPDE_PHASE_STAMPS", 0) ? 1 : 0;
@@ -1215,7 +1220,7 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
     }
     NetArgsHost a = net_args(p);
     GradientPlan g = network_gradients(p, blocks, accumulate, space, a);
-    // the backward half reads the row-major weight copies of every hidden
+    // the launch reads the products' weight operands of every hidden
     // transition, which no workgroup of the same launch may still be writing;
     // RPROP and Adam keep them current between epochs
     if (!n.ws_current) refresh_operands(n);
@@ -1467,7 +1472,7 @@ int cpde_net_create(cpde_device* dev, int layers, const int* neurons, const int*
         for (int t = 0; t < T; ++t) {
             const size_t count = n->param_count(t);
             for (int b = 0; b < 4; ++b) HIP_CHECK(hipMalloc(&n->state[b][t], count * sizeof(float)));
-// the widths that the network-fused kernels take
+            // the widths that the network-fused kernels take
             if (t > 0 && t + 1 < T && n->neurons[t] <= 256 && n->neurons[t + 1] <= 256) {
                 const size_t words = n->split ? weight_operands(n->neurons[t], n->neurons[t + 1]) / 2
                                               : size_t(n->neurons[t]) * n->neurons[t + 1];
@@ -2326,7 +2331,7 @@ int cpde_capture_begin(cpde_device* dev) {
 }
 
 // The recorded calls never ran: their host bookkeeping is undone (active
-// gradient buffers back to the capture's start; the row-major weight copies
+// gradient buffers back to the capture's start; the products' weight operands
 // are rewritten before their next use).
 static void abandon_capture(Device& d) {
     for (auto& c : d.capture_nets) {

@@ -742,6 +742,7 @@ static void emit_prologue(std::ostream& o, const Tables& t, const std::vector<in
     if (tuning.inkernel_wgrad) o << "#define CPDE_INKERNEL_WGRAD 1\n";
     if (tuning.b_pairs) o << "#define CPDE_B_PAIRS 1\n";
     if (tuning.stamps) o << "#define CPDE_STAMPS 1\n";
+    if (tuning.tier_cus) o << "#define CPDE_TIER_CUS " << tuning.tier_cus << "\n";
     // row splits of the compositions used by the network-fused kernels (scaled
     // forward compositions split over mirror lanes instead)
     std::vector<int> splits;
@@ -788,6 +789,7 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    float* const S = T;\n"
        << "#endif\n"
        << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n"
+       << "    tier_raise(a);\n"
        << prefetch << "    const float xin = input_ahead<" << neurons[0] << ">(a, p0, npts);  // for the input gradient\n"
        << "    net_input<" << neurons[0] << ", " << neurons[1] << ", " << operand(L > 3) << ">(a, X, p0, npts);\n"
        << "    __syncthreads();\n"
@@ -807,7 +809,8 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    net_output<" << neurons[L - 2] << ", " << NO << ">(a, " << L - 2 << ", X, p0, npts, O);\n"
        << "    __syncthreads();  // the output values of the block's columns are in O\n"
        << cost << "    net_output_backward<" << neurons[L - 2] << ", " << NO << ", " << operand(L > 3) << ", true>(a, " << L - 2
-       << ", X, p0, npts, ua, O + kNNC * " << NO << ", &wa);\n";
+       << ", X, p0, npts, ua, O + kNNC * " << NO << ", &wa);\n"
+       << "    tier_drop();\n";
     for (int t = L - 3; t >= 1; --t)
         ep << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t > 1)
            << (t == 1 ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
