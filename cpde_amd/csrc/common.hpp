@@ -227,7 +227,7 @@ struct ReduceArgs {
     int splits2[kMaxTransitions];
     int transitions, accumulate, second;
     // cost finishes riding in the launch: one more block finishes them in
-    // order (each as launch_finish_cost would, from at most kMaxCostBlocks
+    // order (each as cost_finish_kernel would, from at most kMaxCostBlocks
     // records), then, with `with_graph`, evaluates the scalar graph on its
     // first lane, which wrote the finished costs
     const CostStats* cost_partials[kReduceCosts];
@@ -467,7 +467,7 @@ inline size_t weight_operands(int n_in, int n_out) {
 void launch_weight_operands(Device& d, const float* const* W, void* const* WS, const int* n_in, const int* n_out,
                             int count, bool split);
 // Fixed-order sum of `blocks` per-workgroup cost records into cost slot cost_index.
-void launch_finish_cost(Device& d, const CostStats* partials, int blocks, int cost_index);
+int launch_stage_cost(Device& d, const CostStats* partials, int blocks, CostStats* out);
 // Zero the slots among [0, count) still marked fresh (before something reads them on the device).
 void launch_clear_fresh(Device& d, int count);
 void launch_fill(Device& d, float* p, size_t count, float value);

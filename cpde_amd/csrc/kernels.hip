@@ -1862,22 +1862,22 @@ __global__ __launch_bounds__(kCostThreads) void cost_stage_kernel(const CostStat
     if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
-void launch_finish_cost(Device& d, const CostStats* partials, int blocks, int cost_index) {
+// More than kMaxCostBlocks records into at most that many at `out`; their number.
+int launch_stage_cost(Device& d, const CostStats* partials, int blocks, CostStats* out) {
+    TraceScope trace(d, kTraceReduce, double(sizeof(CostStats)) * blocks);
+    const int per = (blocks + kMaxCostBlocks - 1) / kMaxCostBlocks;
+    const int staged = (blocks + per - 1) / per;
+    hipLaunchKernelGGL(cost_stage_kernel, staged, kCostThreads, 0, d.stream, partials, blocks, per, out);
+    HIP_CHECK(hipGetLastError());
+    return staged;
+}
+
+static void finish_cost(Device& d, int blocks, int cost_index) {
     TraceScope trace(d, kTraceReduce, double(sizeof(CostStats)) * (blocks + 2));
-    if (blocks > kMaxCostBlocks) {
-        const int per = (blocks + kMaxCostBlocks - 1) / kMaxCostBlocks;
-        const int staged = (blocks + per - 1) / per;
-        hipLaunchKernelGGL(cost_stage_kernel, staged, kCostThreads, 0, d.stream, partials, blocks, per, d.cost_blocks);
-        HIP_CHECK(hipGetLastError());
-        partials = d.cost_blocks;
-        blocks = staged;
-    }
-    hipLaunchKernelGGL(cost_finish_kernel, 1, kCostThreads, 0, d.stream, partials, blocks,
+    hipLaunchKernelGGL(cost_finish_kernel, 1, kCostThreads, 0, d.stream, d.cost_blocks, blocks,
                        d.cost_totals + cost_index, int(d.take_fresh(cost_index)));
     HIP_CHECK(hipGetLastError());
 }
-
-static void finish_cost(Device& d, int blocks, int cost_index) { launch_finish_cost(d, d.cost_blocks, blocks, cost_index); }
 
 __global__ void clear_costs_kernel(CostStats* c, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x) c[i] = empty_cost();

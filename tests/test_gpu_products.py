@@ -65,6 +65,13 @@ def test_long_one_pass_of_narrow_layers(device, variables, order, neurons, point
         run.step()
         device.synchronize()
         got.append((run.loss(), run.gradients()))
+        # deferred, the chunks' reductions finish their staged cost records together
+        hip.check(hip.load().cpde_gradients_defer(device.handle, 1))
+        run.step()
+        assert run.loss() == got[-1][0]
+        hip.check(hip.load().cpde_gradients_defer(device.handle, 0))
+        for a, b in zip(run.gradients(), got[-1][1]):
+            assert np.array_equal(a, b)
         run.plan.stack_ptr(1, 1)
         run.step()
         device.synchronize()
