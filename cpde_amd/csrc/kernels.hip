@@ -492,10 +492,6 @@ __device__ __forceinline__ void wgrad_thin_any(const WgradArgs& a, int t, int sp
     else wgrad_thin(a, t, split, red);
 }
 
-// Workgroups go to the eight XCDs round-robin (workgroup b on XCD b % 8), each
-// XCD with its own L2.  This renumbering gives every XCD a contiguous range of
-// work items, so that the tiles of one split, which read the same rows of G
-// or Y, run under one L2.  It is a permutation of [0, n) for any n.
 // The group whose range [begin[t], begin[t + 1]) holds b (b in [0,
 // begin[count])).  Every boundary is loaded at once and compared, instead of a
 // search whose every step waits on the load before it: kernel arguments come
@@ -508,9 +504,23 @@ __device__ __forceinline__ int group_of(const int (&begin)[kMaxTransitions + 1],
     return t;
 }
 
+// Workgroups go to the eight XCDs round-robin (workgroup b on XCD b % 8), each
+// XCD with its own L2.  This renumbering gives every XCD a contiguous range of
+// work items, so that the tiles of one split, which read the same rows of G
+// or Y, run under one L2.  It is a permutation of [0, n) for any n.
 __device__ __forceinline__ int xcd_grouped(int b, int n) {
     const int x = b & 7, q = b >> 3, per = (n + 7) >> 3, full = (n & 7) ? (n & 7) : 8;
     return x < full ? x * per + q : full * per + (x - full) * (per - 1) + q;
+}
+
+// This workgroup's work item of transition t, renumbered within the transition:
+// a renumbering across the launch gave whole transitions to single XCDs, so
+// that a launch of tiles between thin transitions ran its tiles on two XCDs of
+// eight (3->64^3->1 at order 6 over 2,000 points 129.8 -> 54.2 us, its stacks at
+// the rate of a copy), and so for a second pass's transitions with few columns
+// (the Poisson problem's graph epoch 52.0 -> 49.4 us).
+__device__ __forceinline__ int xcd_item(const WgradArgs& a, int t) {
+    return xcd_grouped(int(blockIdx.x) - a.block_begin[t], a.block_begin[t + 1] - a.block_begin[t]);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -848,9 +858,7 @@ void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a
 __global__ __launch_bounds__(256, 2) void wgrad_grouped_kernel(WgradArgs a) {
     __shared__ __attribute__((aligned(16))) float lds[kWgLds];
     static_assert(256 * 4 * (kThinNarrow + 1) <= kWgLds && 256 * 17 <= kWgLds, "thin-transition scratch exceeds the shared LDS");
-    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
-    const int t = group_of(a.block_begin, a.transitions, b);
-    const int local = b - a.block_begin[t];
+    const int t = group_of(a.block_begin, a.transitions, int(blockIdx.x)), local = xcd_item(a, t);
     if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin_any(a, t, local, lds);
     else if (a.tile[t] == 64) wgrad_tile<64>(a, t, local, lds);
     else wgrad_tile<128>(a, t, local, lds);
@@ -1523,9 +1531,7 @@ __device__ __forceinline__ void wgrad_split_tile(const WgradArgs& a, int t, int 
 __global__ __launch_bounds__(256, CPDE_WD_MIN_BLOCKS) void wgrad_direct_kernel(WgradArgs a) {
     __shared__ __attribute__((aligned(16))) float lds[kWdLds];
     static_assert(256 * 4 * (kThinNarrow + 1) <= kWdLds && 256 * 17 <= kWdLds, "thin-transition scratch exceeds the shared LDS");
-    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
-    const int t = group_of(a.block_begin, a.transitions, b);
-    const int local = b - a.block_begin[t];
+    const int t = group_of(a.block_begin, a.transitions, int(blockIdx.x)), local = xcd_item(a, t);
     if (a.M[t] <= 16 || a.N[t] <= 16) wgrad_thin_any(a, t, local, lds);
     else if (a.M[t] % 4 == 0 && a.N[t] % 4 == 0) wgrad_direct_tile<true>(a, t, local, lds);
     else wgrad_direct_tile<false>(a, t, local, lds);
@@ -1537,9 +1543,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_split_kernel(WgradArgs a) {
     constexpr int kBytes = sp_lds_bytes(256) > 4 * kWdLds ? sp_lds_bytes(256) : 4 * kWdLds;
     __shared__ __attribute__((aligned(16))) unsigned char lds[kBytes];
     float* const floats = reinterpret_cast<float*>(lds);
-    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
-    const int t = group_of(a.block_begin, a.transitions, b);
-    const int local = b - a.block_begin[t];
+    const int t = group_of(a.block_begin, a.transitions, int(blockIdx.x)), local = xcd_item(a, t);
     const bool vec = a.M[t] % 4 == 0 && a.N[t] % 4 == 0;
     if (a.tile[t] == 128) {
         if (vec) wgrad_split_tile<128, true>(a, t, local, lds);
@@ -1553,9 +1557,8 @@ __global__ __launch_bounds__(256, 2) void wgrad_split_kernel(WgradArgs a) {
 template <bool VEC>
 __global__ __launch_bounds__(512, 2) void wgrad_split256_kernel(WgradArgs a) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[sp_lds_bytes(512)];
-    const int b = xcd_grouped(int(blockIdx.x), int(gridDim.x));
-    const int t = group_of(a.block_begin, a.transitions, b);
-    wgrad_split_tile<256, VEC>(a, t, b - a.block_begin[t], lds);
+    const int t = group_of(a.block_begin, a.transitions, int(blockIdx.x));
+    wgrad_split_tile<256, VEC>(a, t, xcd_item(a, t), lds);
 }
 
 // The entries of a whose tile is 256 (or is not), renumbered.
