@@ -530,7 +530,21 @@ static void compose_adjoint(Device& d, const Plan& p, const float* z, float* g, 
     if (!p.rows_module) return launch_compose_adjoint(d, p, z, g, n);
     int elements = p.width * n;
     TraceScope trace(d, kTraceComposeAdjoint, 12.0 * double(elements) * p.rows);
-    void* args[] = {&z, &g, &n, &elements};
+    const float* none = nullptr;
+    int outputs = 0;
+    void* args[] = {&z, &g, &none, &none, &n, &outputs, &elements};
+    launch_module(d, p.rows_module->adjoint, unsigned((elements + 255) / 256), 1, args);
+}
+// dE/dz of the last hidden layer from the output layer's dE/dz, up to
+// kOutputForwardMax outputs: dE/dy, a product of so few terms, is formed on the
+// way into the adjoint instead of through memory (3->64^3->1 at order 6 over
+// 2,000 points 56 -> 35 us of the two launches; 512 -> 1 over 12,288 columns 22 ->
+// 9).
+static void compose_output_adjoint(Device& d, const Plan& p, int t) {
+    Net& n = *p.net;
+    int ni = n.neurons[t], no = n.neurons[t + 1], elements = p.width * ni;
+    TraceScope trace(d, kTraceComposeAdjoint, 8.0 * double(elements) * p.rows);
+    void* args[] = {&n.z[t], &n.g[t], &n.g[t + 1], &n.state[0][t], &ni, &no, &elements};
     launch_module(d, p.rows_module->adjoint, unsigned((elements + 255) / 256), 1, args);
 }
 
@@ -1240,9 +1254,9 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
         launch_module(d, kernel, unsigned(blocks), 1, args, unsigned(p.fused->net_threads));
     }
     // The cost's finish rides in the gradient reduction launch, behind a stage
-    // of its own for more records than one workgroup finishes at once (a finish
-    // launch of its own instead: 2->64^3->1 at order 2 over 16,384 points with Adam 124.1 -> 121.3 us,
-    // 2->50^3->1 at order 3 over 5,003 87.3 -> 83.8).
+    // of its own for more records than one workgroup finishes at once (against a
+    // finish launch of its own: 2->64^3->1 at order 2 over 16,384 points with Adam
+    // 124.1 -> 121.3 us, 2->50^3->1 at order 3 over 5,003 87.3 -> 83.8).
     g.ra.costs = 1;
     g.ra.cost_partials[0] = staged ? staged : records;
     g.ra.cost_total[0] = d.cost_totals + cost_index;
@@ -1905,6 +1919,10 @@ int cpde_backward(cpde_plan* plan, int accumulate) {
         const int cols = int(plan->columns());
         for (int t = n.layers - 2; t >= 1; --t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
+            if (plan->rows_module && t == n.layers - 2 && no <= kOutputForwardMax && !n.linear[t]) {
+                compose_output_adjoint(d, *plan, t);
+                continue;
+            }
             launch_gemm(d, ni, cols, no, n.state[0][t], no, true, n.g[t + 1], no, n.g[t], ni, nullptr, 1);
             if (!n.linear[t]) compose_adjoint(d, *plan, n.z[t], n.g[t], ni);
         }

@@ -523,7 +523,8 @@ std::string compose_source(const Tables& t, const std::vector<int>& splits, bool
 // registers, unscaled stacks on both sides.  rows_forward_k: y from z.
 // rows_adjoint_k: dE/dz from z and dE/dy, in place over the latter; the jet of
 // sigma'(z) is formed again from z, and the adjoint's loads follow it so that
-// z, y and u need not stay live beside dE/dy.
+// z, y and u need not stay live beside dE/dy.  With Gout, the
+// few outputs' adjoints, dE/dy is formed from them and W (as in a linear step).
 std::string rows_source(const Tables& t) {
     const Jet J(t);
     const std::vector<float> fact = row_factorials(J);
@@ -553,18 +554,34 @@ extern "C" __global__ __launch_bounds__(256) void rows_forward_k(const float* __
     for (int r = 0; r < R; ++r) Y[base + size_t(r) * n] = y[r] * kScale[r];
 }
 extern "C" __global__ __launch_bounds__(256) void rows_adjoint_k(const float* __restrict__ Z, float* __restrict__ G,
-                                                                 int n, int elements) {
+                                                                 const float* __restrict__ Gout,
+                                                                 const float* __restrict__ W, int n, int outputs,
+                                                                 int elements) {
     const int e = blockIdx.x * 256 + threadIdx.x;
     if (e >= elements) return;
-    const int p = e / n;
-    const size_t base = size_t(p) * R * n + (e - p * n);
+    const int p = e / n, i = e - p * n;
+    const size_t base = size_t(p) * R * n + i;
     float z[R], y[R], u[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) z[r] = Z[base + size_t(r) * n] * kUnscale[r];
     compose(z, y, u);
     float gy[R], gz[R];
+    if (Gout) {
+        const float* g = Gout + size_t(p) * R * outputs;
 #pragma unroll
-    for (int r = 0; r < R; ++r) gy[r] = G[base + size_t(r) * n] * kScale[r];
+        for (int r = 0; r < R; ++r) gy[r] = 0.0f;
+#pragma unroll 1
+        for (int o = 0; o < outputs; ++o) {
+            const float w = W[o + outputs * i];
+#pragma unroll
+            for (int r = 0; r < R; ++r) gy[r] = fmaf(w, g[r * outputs + o], gy[r]);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) gy[r] = G[base + size_t(r) * n];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) gy[r] *= kScale[r];
     adjoint(u, gy, gz);
 #pragma unroll
     for (int r = 0; r < R; ++r) G[base + size_t(r) * n] = gz[r] * kUnscale[r];

@@ -18,6 +18,7 @@ SHAPES = [
     (2, 2, [2, 264, 257, 1], 29, 13),
     (1, 0, [1, 300, 1], 5, 0),
     (2, 6, [2, 288, 31, 1], 1, 0),
+    (3, 6, [3, 17, 65, 1], 6, 0),
 ]
 
 
@@ -55,3 +56,31 @@ def test_row_kernel_epoch_matches_oracle(device, monkeypatch, variables, order, 
     assert abs(loss / table_loss - 1) < 1e-5
     for t, (g, w) in enumerate(zip(grads, table)):
         assert rel_l2(g, w) < 1e-4, t
+
+
+@pytest.mark.parametrize('outputs', [1, 3, 8, 9])   # up to 8 the output adjoint forms dE/dy itself
+def test_output_adjoint_of_row_kernels(device, monkeypatch, outputs):
+    """Gradients from given dE/dz of the output layer, against the table-driven
+    path, whose products run on their own."""
+    neurons, points = [2, 270, outputs], 7
+    print(f'[case] output adjoint, {outputs} outputs', flush=True)
+    schema = W.full_schema(2, 3)
+    init = W.xavier_weights(neurons, 5)
+    pts = np.random.default_rng(5).random((points, 2), dtype=np.float32)
+    stack = np.ascontiguousarray(W.input_stack(pts, schema).transpose(0, 2, 1), np.float32)
+    adjoint = np.random.default_rng(6).standard_normal(points * len(schema) * outputs).astype(np.float32)
+    got = []
+    for fused in ('2', '0'):
+        monkeypatch.setenv('CPDE_FUSED', fused)
+        net = hip.Net(device, neurons, W.linear_flags(neurons), init)
+        plan = hip.Plan(net, schema, points, True)
+        data = hip.Buffer.of(device, stack)
+        plan.activate(data, points, np.arange(len(schema), dtype=np.int32), 0, points)
+        plan.forward()
+        device.upload_ptr(plan.stack_ptr(2, 2), adjoint)
+        plan.backward(False)
+        got.append([net.gradient(t) for t in range(2)])
+        data.free()
+        plan.destroy(); net.destroy()
+    for t in range(2):
+        assert rel_l2(got[0][t], got[1][t]) < 1e-5, t
