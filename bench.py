@@ -53,22 +53,22 @@ MFMA_KINDS = {'gemm_forward', 'gemm_transposed', 'gemm_wgrad', 'fused_forward', 
 CPU_SAMPLE_MACS = 3.0e9
 
 # HBM bytes per launch from rocprofv3 counter passes over this benchmark
-# (profiles/network_kernels_<workload>_traffic.md and _counters.md): mean FETCH_SIZE and
+# (profiles/network_kernels_traffic.md; poisson_disk_order2: _counters.md): mean FETCH_SIZE and
 # WRITE_SIZE in KiB per dispatch, scaled by what the same counters read for a
 # plain 256 MiB copy (``--copy-calibration``): 268,435,456 B / 131,084.475 KiB
 # read, 268,435,456 B / 262,144 KiB written.
 COPY_SCALE = (268435456 / (131084.475 * 1024), 268435456 / (262144 * 1024))
 TRAFFIC_KIB = {
-    'fourier_fit_order2': {'network_epoch': (5101.3, 30162.8), 'gemm_wgrad': (6878.0, 3898.0),
-                           'split_reduce': (3952.1, 2713.1)},
-    'fourier_fit_order6': {'network_epoch': (20859.94, 134919.15), 'gemm_wgrad': (31754.55, 4077.5),
-                           'split_reduce': (4544.0, 2713.12)},
+    'fourier_fit_order2': {'network_epoch': (5843.1, 25788.75), 'gemm_wgrad': (7327.5, 3954.0),
+                           'split_reduce': (3974.35, 4377.12)},
+    'fourier_fit_order6': {'network_epoch': (18758.46, 113939.95), 'gemm_wgrad': (34724.46, 4147.5),
+                           'split_reduce': (4561.9, 4377.12)},
     'poisson_disk_order2': {'network_epoch': (6934.3, 54427.2), 'gemm_wgrad': (7005.0, 2946.7),
                             'split_reduce': (1940.5, 261.7)},
-    'fourier_3d_order4': {'network_forward': (51367.6, 5739531.1), 'network_backward': (1753565.2, 3341379.0),
-                          'gemm_wgrad': (2329450.2, 4388.1), 'split_reduce': (22647.6, 1113.0)},
-    'fourier_large_order6': {'network_backward': (4986651.81, 8870448.64), 'network_forward': (423199.55, 14688002.1),
-                             'gemm_wgrad': (6994723.69, 4064.13)},
+    'fourier_3d_order4': {'network_forward': (102824.02, 5739264.75), 'network_backward': (1827527.51, 3215728.27),
+                          'gemm_wgrad': (2326641.64, 33273.6), 'split_reduce': (37114.11, 1120.4)},
+    'fourier_large_order6': {'network_backward': (5195012.63, 8391610.28), 'network_forward': (602051.27, 14687232.0),
+                             'gemm_wgrad': (5603621.21, 66699.63)},
 }
 
 

@@ -517,7 +517,7 @@ constexpr int kOutputForwardMax = 8;
 // kernels on unscaled stacks), bound by the stacks' bytes; the table-driven
 // kernels walk every partition of every row from memory.  3->64^3->1 at order 6
 // (84 rows) over 2,000 points, a layer's adjoint 833 -> 39 us (3.3 TB/s at one
-// wave per SIMD) and forward 381 -> under 20 us, the epoch 4,226 -> 731 us;
+// wave per SIMD; 31 now) and forward 381 -> under 20 us, the epoch 4,226 -> 731 us;
 // 2->512^3->1 at order 2, 2,048-point chunks, 26 -> 12 and 17 -> 9 us.
 static void compose_forward(Device& d, const Plan& p, const float* z, float* y, int n) {
     if (!p.rows_module) return launch_compose_forward(d, p, z, y, n);
@@ -538,8 +538,8 @@ static void compose_adjoint(Device& d, const Plan& p, const float* z, float* g, 
 // dE/dz of the last hidden layer from the output layer's dE/dz, up to
 // kOutputForwardMax outputs: dE/dy, a product of so few terms, is formed on the
 // way into the adjoint instead of through memory (3->64^3->1 at order 6 over
-// 2,000 points 56 -> 35 us of the two launches; 512 -> 1 over 12,288 columns 22 ->
-// 9).
+// 2,000 points, three layers' adjoints and the product 139 -> 93 us, the gradient
+// 383 -> 338; 2->512^3->1 at order 2 in 2,048-point chunks 805 -> 788).
 static void compose_output_adjoint(Device& d, const Plan& p, int t) {
     Net& n = *p.net;
     int ni = n.neurons[t], no = n.neurons[t + 1], elements = p.width * ni;
