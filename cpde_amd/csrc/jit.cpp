@@ -784,7 +784,7 @@ static const char* operand(bool yes) { return yes ? "true" : "false"; }
 // Body of a one-pass epoch kernel: the forward of the workgroup's points, the
 // output values and the output adjoint of its columns kept in LDS (O), the
 // cost stage `cost` between them (it fills O's second half), then the
-// backward.  The row-major weight copies are written before the launch.
+// backward.  The products' weight operands are written before the launch.
 static std::string epoch_body(const std::vector<int>& neurons, const std::string& prefetch, const std::string& cost,
                               const FusedTuning& tuning, const std::string& after_input = "") {
     const int L = int(neurons.size()), NO = neurons[L - 1];
