@@ -331,9 +331,22 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
         bool paired = rows > 16 && width >= 16 * compute_units && neurons.size() >= 3;
         for (size_t l = 1; l + 1 < neurons.size(); ++l) paired = paired && neurons[l] > 64 && neurons[l] % 16 == 0;
         if (paired) {
-            npb = 2;
-            t.alias = 1;
-            t.col_tile = 16;
+            FusedTuning pair;
+            pair.net_points_per_block = 2;
+            pair.alias = 1;
+            pair.col_tile = 16;
+            pair.max_split = 1;  // one tile needs whole columns per lane, of a layer beside a wider one too
+            // Split products of layers wider than 128 leave room for one workgroup
+            // per CU: eight waves (2->256^4->1, order 6: 74.5 -> 68.1 ms per epoch).
+            if (split_products(neurons) && *std::max_element(neurons.begin() + 1, neurons.end() - 1) > 128)
+                pair.net_threads = 512;
+            // Split operands are half as large again as fp32 ones: 56 rows of
+            // 208-wide layers and eight outputs fit one point at a time (3->208^3->8
+            // over 8,192 points 4.28 ms per epoch, on pairs of fp32 operands 6.09).
+            if (network_lds(rows, neurons, pair) <= kLdsBytes) {
+                t = pair;
+                npb = 2;
+            }
         }
     }
     // A value-only plan over at most one point per CU (a boundary leaf, which
@@ -356,9 +369,6 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // CUs it was slower (order 4, 365 workgroups: 0.0700 -> 0.0742).
     if (width > 0 && rows <= 16 && npb > 1 && !value_leaf && (width + npb - 1) / npb <= compute_units)
         t.net_threads = 512;
-    // Two points of layers wider than 128 leave room for one workgroup per CU:
-    // eight waves (2->256^4->1, order 6: 74.5 -> 68.1 ms per epoch).
-    if (t.alias && *std::max_element(neurons.begin(), neurons.end()) > 128) t.net_threads = 512;
     t.net_threads = env_int("CPDE_NET_THREADS", t.net_threads) == 512 ? 512 : 256;
     // The waves of a workgroup share a layer's fp32 products by output tile.  Where
     // 32x32 tiles of the narrowest hidden layer are fewer than the waves (a
@@ -404,8 +414,7 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     t.scaled = env_int("CPDE_SCALED", t.scaled) ? 1 : 0;
     // Wave priorities by dispatch round (tier_raise in the generated source).
     const int blocks = (width + t.net_points_per_block - 1) / t.net_points_per_block;
-    if (env_int("CPDE_NET_TIERS", 1) && !split_products(neurons) && blocks > compute_units &&
-        resident(blocks, compute_units))
+    if (env_int("CPDE_NET_TIERS", 1) && widest < 128 && blocks > compute_units && resident(blocks, compute_units))
         t.tier_cus = compute_units;
     // Diagnostics: clock stamps of the one-pass epoch's phases, written over
     // the output stack (cpde_amd/stamps.py reads them back).

@@ -407,6 +407,10 @@ struct FusedTuning {
     int tier_cus = 0;              // one-pass epochs: wave priorities by dispatch round on this many CUs (0: none)
     int stamps = 0;                // one-pass epochs write per-phase clock stamps over their output stack
 };
+// Bytes of LDS that a workgroup of the network kernels takes at most, for a
+// schema of `rows` rows (with tuning.alias: as one LDS tile), and what it may take.
+size_t network_lds(int rows, const std::vector<int>& neurons, const FusedTuning& tuning);
+constexpr size_t kLdsBytes = 160 * 1024;
 // Whether the schema is closed under swapping variables 0 and 1 (the scaled
 // forward composition then splits over two lanes, one per mirror image).
 bool mirror_symmetric(const Tables& t);

@@ -685,11 +685,48 @@ static int forward_split_cap(const Tables& t, const FusedTuning& tuning) {
     return mirror_symmetric(t) ? std::min(tuning.max_split, 2) : 1;
 }
 
-// Whether a network's products run on split bf16 operands (fused.hip.in).
+// Whether a network's products run on split bf16 operands (fused.hip.in); a
+// single hidden layer has none.
 bool split_products(const std::vector<int>& neurons) {
-    int widest = 0;
-    for (size_t l = 1; l + 1 < neurons.size(); ++l) widest = std::max(widest, neurons[l]);
-    return widest >= 128;
+    return neurons.size() > 3 && *std::max_element(neurons.begin() + 1, neurons.end() - 1) >= 128;
+}
+
+namespace {
+
+int widest_hidden(const std::vector<int>& neurons) {
+    return *std::max_element(neurons.begin() + 1, neurons.end() - 1);
+}
+// Row strides of the LDS tiles: floats of a product's columns, bf16s of an operand plane.
+int tile_stride(int widest) { return (widest + 7) / 8 * 8 + 4; }
+int plane_stride(int widest) { return (widest + 31) / 32 * 32 + 8; }
+
+// Column tile of the fp32 network products (the split ones take 16): 16 (v_mfma_f32_16x16x4f32) or 32
+// (v_mfma_f32_32x32x2f32), as the tuning chose it; without a choice, 16 when
+// a block holds one point.  16 needs every hidden width a multiple of 16.
+// Measured on 2->128^4->1 at 729 points, epoch kernel: one point per block
+// (orders 5, 6; 21 and 28 rows) 16 is 6 and 2 % faster, and 35 rows pad to
+// 48 columns instead of 64 (3D order 4: 11 %).
+int column_tile(const std::vector<int>& neurons, const FusedTuning& tuning) {
+    if (split_products(neurons)) return 16;
+    for (size_t l = 1; l + 1 < neurons.size(); ++l)
+        if (neurons[l] % 16) return 32;
+    if (tuning.col_tile == 16 || tuning.col_tile == 32) return tuning.col_tile;
+    return tuning.net_points_per_block == 1 ? 16 : 32;
+}
+
+}  // namespace
+
+// The one-pass epoch's arrays, which include the other network kernels': the
+// tiles X and T (tile_declarations), O, S and the input stack ahead (epoch_body,
+// net_input_gradient).
+size_t network_lds(int rows, const std::vector<int>& neurons, const FusedTuning& tuning) {
+    const int widest = widest_hidden(neurons), tile = column_tile(neurons, tuning);
+    const size_t used = size_t(tuning.net_points_per_block) * rows, columns = (used + tile - 1) / tile * tile;
+    const size_t products = 4 * columns * tile_stride(widest), outputs = 4 * columns * neurons.back();
+    size_t bytes = std::max(products, split_products(neurons) ? 6 * columns * plane_stride(widest) : 0);
+    bytes += tuning.alias ? std::max<size_t>(outputs, 16 * tuning.net_points_per_block) : products;
+    const size_t input = used * neurons[0];
+    return bytes + 2 * outputs + (input <= size_t(tuning.net_threads) ? 4 * input : 4) + 64;  // rounding of each array
 }
 
 // Whether every hidden layer's forward and adjoint compositions have one lane
@@ -720,39 +757,21 @@ static void emit_prologue(std::ostream& o, const Tables& t, const std::vector<in
                           const FusedTuning& tuning) {
     const int points_per_block = tuning.points_per_block, net_points_per_block = tuning.net_points_per_block;
     const int L = int(neurons.size());
-    int widest = 0;
-    for (int l = 1; l + 1 < L; ++l) widest = std::max(widest, neurons[l]);
+    const int widest = widest_hidden(neurons);
     o << "// generated: cPDE layer-fused kernels\n#define CPDE_POINTS " << points_per_block << "\n";
     o << "#define CPDE_NET_POINTS " << net_points_per_block << "\n";
     o << "#define CPDE_NET_THREADS " << tuning.net_threads << "\n";
-    o << "#define CPDE_STRIDE " << ((widest + 7) / 8 * 8 + 4) << "\n";
-    // Column tile of the fp32 network products (the split ones take 16): 16 (v_mfma_f32_16x16x4f32) or 32
-    // (v_mfma_f32_32x32x2f32), as the tuning chose it; without a choice, 16 when
-    // a block holds one point.  16 needs every hidden width a multiple of 16.
-    // Measured on 2->128^4->1 at 729 points, epoch kernel: one point per block
-    // (orders 5, 6; 21 and 28 rows) 16 is 6 and 2 % faster, and 35 rows pad to
-    // 48 columns instead of 64 (3D order 4: 11 %).
-    {
-        bool hidden16 = true;
-        for (int l = 1; l + 1 < L; ++l) hidden16 = hidden16 && neurons[l] % 16 == 0;
-        int col_tile = net_points_per_block == 1 ? 16 : 32;
-        if (tuning.col_tile == 16 || tuning.col_tile == 32) col_tile = tuning.col_tile;
-        if (!hidden16) col_tile = 32;
-        if (split_products(neurons)) col_tile = 16;
-        o << "#define CPDE_COL_TILE " << col_tile << "\n";
-    }
+    o << "#define CPDE_STRIDE " << tile_stride(widest) << "\n";
+    o << "#define CPDE_COL_TILE " << column_tile(neurons, tuning) << "\n";
     if (split_products(neurons)) o << "#define CPDE_SPLIT_PRODUCTS 1\n";
-    o << "#define CPDE_PLANE_STRIDE " << ((widest + 31) / 32 * 32 + 8) << "\n";
+    o << "#define CPDE_PLANE_STRIDE " << plane_stride(widest) << "\n";
     const int forward_cap = forward_split_cap(t, tuning);
     o << "#define CPDE_MAX_SPLIT " << forward_cap << "\n";
-    // One LDS tile instead of two when every composition has whole columns per
+    // One LDS tile instead of two, where every composition has whole columns per
     // lane (no split): every lane takes its columns' z rows before any writes
     // its y rows over them, and the products wait for every wave's operand
-    // reads before they store.  Two fifths less LDS per workgroup: on request,
-    // or where two tiles would pass the workgroup's 160 KB.
-    const int columns = (net_points_per_block * t.rows + 15) / 16 * 16;
-    const size_t tile_bytes = size_t(columns) * (6 * ((widest + 31) / 32 * 32 + 8) + 4 * ((widest + 7) / 8 * 8 + 4));
-    if ((tuning.alias || (split_products(neurons) && tile_bytes > 150 * 1024)) && alias_tiles(t, neurons, tuning))
+    // reads before they store.  Two fifths less LDS per workgroup.
+    if (tuning.alias && alias_tiles(t, neurons, tuning))
         o << "#define CPDE_ALIAS_TILES 1\n";
     o << "#define CPDE_MAX_SPLIT_ADJOINT " << tuning.max_split_adjoint << "\n";
     if (tuning.scaled) o << "#define CPDE_SCALED 1\n";
