@@ -23,6 +23,7 @@ struct cpde_replay_s {
         cpde::Net* net;
         std::vector<int> before, after;  // active gradient buffers when recorded, and after the recording
         uint64_t generation;
+        bool forward;  // whether it runs a forward on the network's arena
     };
     std::vector<NetState> nets;
 };
@@ -582,9 +583,17 @@ static void refresh_operands(Net& n) {
     n.ws_current = true;
 }
 
+// A forward on the network's arena (not on a bound set's stacks) begins.
+static void arena_forward(Net& n) {
+    if (n.bound) return;
+    ++n.forwards;
+    n.values_only = nullptr;
+}
+
 static void fused_forward(Plan& p) {
     Net& n = *p.net;
     Device& d = *n.dev;
+    arena_forward(n);
     FusedModule& fm = *p.fused;
     const int L = n.layers, R = p.rows;
     int width = p.width;
@@ -599,11 +608,12 @@ static void fused_forward(Plan& p) {
         // A plan without a backward writes its outputs alone: nothing reads the
         // layers' stacks, which are most of such a forward's bytes (65,536 points
         // 2->128^4->1 83 -> 54 us; 10 rows of 32,768 points 3->128^5->1 470 -> 293).
-        const bool values = !p.backward && !n.stacks_out && !n.bound;
+        // (A recording writes every stack: their pointers may go out after it.)
+        const bool values = !p.backward && !n.stacks_out && !n.bound && !d.capturing;
         launch_module(d, values ? fm.network_values : fm.network_forward,
                       unsigned((width + fm.net_points_per_block - 1) / fm.net_points_per_block), 1, args,
                       unsigned(fm.net_threads));
-        n.values_only = values ? &p : nullptr;
+        if (values) n.values_only = &p;
         if (!values) n.ws_current = true;  // fp32 products: written by the forward's side job
         return;
     }
@@ -1227,7 +1237,6 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
     int width = p.width;
     const double cols = double(p.columns());
     const int blocks = epoch_blocks(p);
-    n.values_only = nullptr;
     // a held epoch this one cannot join goes out before anything of this one
     if (d.held && d.held->open && (!program || !epoch_pairs() || d.held->plan == &p || d.held->plan->net != &n))
         flush_held(d);
@@ -1246,6 +1255,7 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
             else flush_wgrad(d);
         }
     }
+    if (!own.on) arena_forward(n);
     NetArgsHost a = net_args(p);
     GradientPlan g = network_gradients(p, blocks, accumulate, space, a);
     // the launch reads the products' weight operands of every hidden
@@ -1758,7 +1768,7 @@ int cpde_forward(cpde_plan* plan) {
             fused_forward(*plan);
             return;
         }
-        n.values_only = nullptr;
+        arena_forward(n);
         const int cols = int(plan->columns());
         for (int t = 0; t + 1 < n.layers; ++t) {
             const int ni = n.neurons[t], no = n.neurons[t + 1];
@@ -2355,7 +2365,7 @@ int cpde_capture_begin(cpde_device* dev) {
         require(!dev->tracing, "tracing times every launch with events; a capture cannot hold them");
         flush_reduce(*dev);
         dev->capture_nets.clear();
-        for (Net* n : dev->nets) dev->capture_nets.push_back({n, n->active});
+        for (Net* n : dev->nets) dev->capture_nets.push_back({n, n->active, n->forwards, n->values_only});
         dev->capture_layout = dev->layout;
         HIP_CHECK(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
         dev->capturing = true;
@@ -2363,12 +2373,13 @@ int cpde_capture_begin(cpde_device* dev) {
 }
 
 // The recorded calls never ran: their host bookkeeping is undone (active
-// gradient buffers back to the capture's start; the products' weight operands
-// are rewritten before their next use).
+// gradient buffers and the arena's state back to the capture's start; the
+// products' weight operands are rewritten before their next use).
 static void abandon_capture(Device& d) {
     for (auto& c : d.capture_nets) {
         c.net->active = c.active;
         c.net->ws_current = false;
+        c.net->values_only = c.values_only;
     }
     d.capture_nets.clear();
 }
@@ -2401,19 +2412,17 @@ int cpde_capture_end(cpde_device* dev, int keep, cpde_replay** out) {
         r->dev = dev;
         r->exec = exec;
         r->layout = dev->layout;
-        for (auto& c : dev->capture_nets) r->nets.push_back({c.net, c.active, c.net->active, c.net->generation});
-        dev->capture_nets.clear();
+        for (auto& c : dev->capture_nets)
+            r->nets.push_back({c.net, c.active, c.net->active, c.net->generation, c.net->forwards != c.forwards});
         // the recorded calls have done their host bookkeeping: their device
         // work runs now
         const hipError_t launched = hipGraphLaunch(exec, dev->stream);
         if (launched != hipSuccess) {
             (void)hipGraphExecDestroy(exec);
-            for (auto& c : r->nets) {
-                c.net->active = c.before;
-                c.net->ws_current = false;
-            }
+            abandon_capture(*dev);
             HIP_CHECK(launched);
         }
+        dev->capture_nets.clear();
         *out = r.release();
     });
 }
@@ -2432,7 +2441,10 @@ int cpde_replay_launch(cpde_replay* replay) {
         for (const auto& c : replay->nets)
             if (!c.net->ws_current) refresh_operands(*c.net);
         HIP_CHECK(hipGraphLaunch(replay->exec, d.stream));
-        for (const auto& c : replay->nets) c.net->active = c.after;
+        for (const auto& c : replay->nets) {
+            c.net->active = c.after;
+            if (c.forward) arena_forward(*c.net);
+        }
     });
 }
 

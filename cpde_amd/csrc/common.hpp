@@ -124,8 +124,10 @@ struct Net {
     // without a backward write every stack, and epochs over more workgroups than
     // fit on the device together stay separate launches, which do
     bool stacks_out = false;
-    // the plan whose forward ran last on the arena, where it wrote no stacks
+    // the plan whose forward ran last on the arena, where it wrote no stacks,
+    // and the forwards that ran there (the recorded ones as they are recorded)
     const struct Plan* values_only = nullptr;
+    uint64_t forwards = 0;
     // split-K partial buffer for the weight-gradient contraction
     float* partials = nullptr;
     size_t partial_capacity = 0;
@@ -333,6 +335,8 @@ struct Device {
     struct NetCapture {
         Net* net;
         std::vector<int> active;
+        uint64_t forwards;
+        const Plan* values_only;
     };
     std::vector<NetCapture> capture_nets;  // state when the open capture began
     // Deferred gradient reductions (cpde_gradients_defer): a backward pass's
