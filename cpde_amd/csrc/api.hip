@@ -304,10 +304,23 @@ struct NetArgsHost {
     void* WS[32];
     float* partial_hidden[32];
     int block_offset, block_count;  // the pass's workgroups in the launch (count 0: the whole grid)
+    int keep;
 };
 
 // Whether a grid's workgroups are all on the device at once (four per CU).
 static bool resident(int blocks, int compute_units) { return blocks <= 4 * compute_units; }
+
+// Whether matching epochs of a network run in one pass over longer grids too:
+// where no hidden layer is wider than 64.  Workgroups that narrow stay many per
+// CU with the backward's registers too, so the forward alone gains nothing, and
+// the kernel saves the cost launch, two stacks and u's way through memory.
+// Epochs, separate -> one pass: 2->50^3->1 at order 3 over 5,003 points 81 -> 72 us,
+// 2->64^3->1 at order 2 over 16,384 131 -> 120, at order 0 over 200,000 377 -> 262,
+// 2->48^3->1 at order 6 over 8,000 250 -> 224; wider: 2->96^3->1 at order 4 over
+// 20,000 616 -> 633, 2->256^3->1 at order 2 over 30,000 1,594 -> 1,663.
+static bool one_pass_any_length(const std::vector<int>& neurons) {
+    return *std::max_element(neurons.begin() + 1, neurons.end() - 1) <= 64;
+}
 
 // Tuning of the fused kernels for a schema of `rows` derivative rows over chunks
 // of `width` points (0: unknown) on `compute_units` CUs, for a network of
@@ -417,6 +430,7 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     const int blocks = (width + t.net_points_per_block - 1) / t.net_points_per_block;
     if (env_int("CPDE_NET_TIERS", 1) && widest < 128 && blocks > compute_units && resident(blocks, compute_units))
         t.tier_cus = compute_units;
+    t.keep_asked = one_pass_any_length(neurons) && !resident(blocks, compute_units);
     // Diagnostics: clock stamps of the one-pass epoch's phases, written over
     // the output stack (cpde_amd/stamps.py reads them back).
     t.stamps = env_int("CPDE_PHASE_STAMPS", 0) ? 1 : 0;
@@ -1029,20 +1043,10 @@ static bool one_pass_fits(const Plan& p) {
     return env_int("CPDE_ONE_PASS", 1) && p.fused && p.network && resident(epoch_blocks(p), p.net->dev->compute_units);
 }
 
-// Whether a matching epoch runs in one pass: also over longer grids, where no
-// hidden layer is wider than 64 (and nobody holds a stack that it leaves
-// unwritten).  Workgroups that narrow stay many per CU with the backward's
-// registers too, so the forward alone gains nothing, and the kernel saves the
-// cost launch, two stacks and u's way through memory.  Epochs, separate -> one
-// pass: 2->50^3->1 at order 3 over 5,003 points 81 -> 72 us, 2->64^3->1 at order 2
-// over 16,384 131 -> 120, at order 0 over 200,000 377 -> 262, 2->48^3->1 at order 6
-// over 8,000 250 -> 224; wider: 2->96^3->1 at order 4 over 20,000 616 -> 633,
-// 2->256^3->1 at order 2 over 30,000 1,594 -> 1,663.
+// Whether a matching epoch runs in one pass.
 static bool matching_one_pass(const Plan& p) {
-    if (one_pass_fits(p)) return true;
-    if (!env_int("CPDE_ONE_PASS", 1) || !p.fused || !p.network || p.net->stacks_out) return false;
-    const std::vector<int>& n = p.net->neurons;
-    return *std::max_element(n.begin() + 1, n.end() - 1) <= 64;
+    return one_pass_fits(p) ||
+           (env_int("CPDE_ONE_PASS", 1) && p.fused && p.network && one_pass_any_length(p.net->neurons));
 }
 
 // The per-workgroup cost records of a one-pass epoch.
@@ -1257,6 +1261,8 @@ static void one_pass_epoch(Plan& p, hipFunction_t kernel, void* cost_args, CostS
     }
     if (!own.on) arena_forward(n);
     NetArgsHost a = net_args(p);
+    // (a recording's stacks may be asked for after it)
+    a.keep = n.stacks_out || d.capturing;
     GradientPlan g = network_gradients(p, blocks, accumulate, space, a);
     // the launch reads the products' weight operands of every hidden
     // transition, which no workgroup of the same launch may still be writing;

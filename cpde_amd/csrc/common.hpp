@@ -121,8 +121,8 @@ struct Net {
     std::vector<size_t> capacity;     // floats per layer buffer
     uint64_t generation = 0;
     // a caller holds a stack's pointer (cpde_plan_stack): from then on forwards
-    // without a backward write every stack, and epochs over more workgroups than
-    // fit on the device together stay separate launches, which do
+    // without a backward write every stack, and so do one-pass epochs over more
+    // workgroups than fit on the device together
     bool stacks_out = false;
     // the plan whose forward ran last on the arena, where it wrote no stacks,
     // and the forwards that ran there (the recorded ones as they are recorded)
@@ -409,6 +409,7 @@ struct FusedTuning {
     int scaled = 1;                // network kernels keep Taylor-scaled sigmoid stacks (row alpha / alpha!)
     int inkernel_wgrad = 0;        // network backward kernels write hidden weight-gradient partials themselves
     int tier_cus = 0;              // one-pass epochs: wave priorities by dispatch round on this many CUs (0: none)
+    int keep_asked = 0;            // one-pass epochs write the stacks that no later launch reads when asked to
     int stamps = 0;                // one-pass epochs write per-phase clock stamps over their output stack
 };
 // Bytes of LDS that a workgroup of the network kernels takes at most, for a

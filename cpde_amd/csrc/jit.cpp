@@ -833,9 +833,10 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
     // the last hidden layer's y (read from X by the output layer's partial) and
     // the first one's dE/dz (read from X by the input transition's) stay in the
     // workgroup: no later launch reads them
+    const std::string unread = tuning.keep_asked ? ", kAsked" : ", kDropped";
     for (int t = 1; t + 2 < L; ++t)
         ep << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
-           << (t + 3 == L ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+           << (t + 3 == L ? unread : "") << ">(a, " << t << ", X, T, p0, npts);\n";
     const std::string last = std::to_string(neurons[L - 2]);
     ep << "    UAhead<" << last << ", output_adjoint_split<" << last
        << ">()> ua;  // the last hidden layer's u rows, in flight during the output layer and the cost\n"
@@ -849,7 +850,7 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    tier_drop();\n";
     for (int t = L - 3; t >= 1; --t)
         ep << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t > 1)
-           << (t == 1 ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+           << (t == 1 ? unread : "") << ">(a, " << t << ", X, T, p0, npts);\n";
     ep << "    net_input_gradient<" << neurons[0] << ", " << neurons[1] << ", true>(a, X, p0, npts, xin);\n";
     // Diagnostics (FusedTuning::stamps): a clock stamp after every phase --
     // each call above and each barrier between them -- written over the
@@ -899,7 +900,7 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
         << "    __syncthreads();\n";
     for (int t = 1; t + 2 < L; ++t)
         val << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
-            << ", false, false>(a, " << t << ", X, T, p0, npts);\n";
+            << ", kDropped, false>(a, " << t << ", X, T, p0, npts);\n";
     val << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
     {
         const std::string last = std::to_string(neurons[L - 2]);

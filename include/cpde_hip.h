@@ -200,8 +200,8 @@ int cpde_cost_matching(cpde_plan* plan, const float* target, int target_width, c
  * activated.  That one launch leaves two stacks unwritten, which no later
  * launch reads: y of the last hidden layer and dE/dz of the first
  * (cpde_plan_stack kinds 1 and 2); read them after the separate calls instead.
- * (Chunks of more workgroups than fit together run as the separate calls, and
- * write them, once a stack's pointer has been asked for on the network.) */
+ * (Chunks of more workgroups than fit together write them too once a stack's
+ * pointer has been asked for on the network, and in every recording.) */
 int cpde_epoch_matching(cpde_plan* plan, const float* target, int target_width, const int* target_rows,
                         const float* weights, int weight_samples, int offset, int valid, int cost_index, int collect,
                         int accumulate);
