@@ -23,7 +23,9 @@ struct cpde_replay_s {
         cpde::Net* net;
         std::vector<int> before, after;  // active gradient buffers when recorded, and after the recording
         uint64_t generation;
-        bool forward;  // whether it runs a forward on the network's arena
+        // whether it runs a forward on the network's arena, and whether stacks of
+        // an earlier one were wanted while it was recorded
+        bool forward, wanted;
     };
     std::vector<NetState> nets;
 };
@@ -305,6 +307,7 @@ struct NetArgsHost {
     float* partial_hidden[32];
     int block_offset, block_count;  // the pass's workgroups in the launch (count 0: the whole grid)
     int keep;
+    float* kept;
 };
 
 // Whether a grid's workgroups are all on the device at once (four per CU).
@@ -526,6 +529,7 @@ static NetArgsHost net_args(const Plan& p) {
         a.G[l] = n.g[l];
     }
     a.X = p.input;
+    a.kept = p.kept;
     a.Z[0] = p.input;
     return a;
 }
@@ -577,23 +581,28 @@ struct PartialSpace;
 static GradientPlan network_gradients(Plan& p, int blocks, bool accumulate, const PartialSpace& space,
                                       NetArgsHost& a);
 
+static int epoch_blocks(const Plan& p);
+
 // Mode of the fused path: CPDE_FUSED=2 (default) network-fused, 1 layer-fused.
 static bool network_mode() { return env_int("CPDE_FUSED", 2) >= 2; }
 
 // Rewrite the product operands of every hidden transition from the weights
-// (one launch).
-static void refresh_operands(Net& n) {
+// `weights` (one launch).
+static void refresh_operands(Net& n, const float* const* weights) {
     std::vector<const float*> W;
     std::vector<void*> WS;
     std::vector<int> ni, no;
     for (int t = 1; t + 2 < n.layers; ++t) {
         if (!n.ws[t]) continue;
-        W.push_back(n.state[0][t]);
+        W.push_back(weights[t]);
         WS.push_back(n.ws[t]);
         ni.push_back(n.neurons[t]);
         no.push_back(n.neurons[t + 1]);
     }
     if (!W.empty()) launch_weight_operands(*n.dev, W.data(), WS.data(), ni.data(), no.data(), int(W.size()), n.split);
+}
+static void refresh_operands(Net& n) {
+    refresh_operands(n, n.state[0].data());
     n.ws_current = true;
 }
 
@@ -602,6 +611,47 @@ static void arena_forward(Net& n) {
     if (n.bound) return;
     ++n.forwards;
     n.values_only = nullptr;
+}
+
+void keep_weights(Net& n) {
+    if (!n.values_only || n.weights_kept || n.dev->capturing) return;  // (a capture: before the recording runs)
+    float* kept = n.values_only->kept + n.values_only->columns() * n.neurons[0];
+    for (int t = 0; t + 2 < n.layers; ++t) {
+        HIP_CHECK(hipMemcpyAsync(kept, n.state[0][t], n.param_count(t) * sizeof(float), hipMemcpyDeviceToDevice,
+                                 n.dev->stream));
+        kept += n.param_count(t);
+    }
+    n.weights_kept = true;
+}
+
+// Somebody is to read the arena's stacks: the last forward's, if it wrote its
+// outputs alone, are written now, from the inputs and weights that it ran on.
+// During a capture they are written before the recording runs.
+static void settle_arena(Net& n) {
+    if (!n.values_only || n.bound) return;
+    Device& d = *n.dev;
+    if (d.capturing) {
+        n.arena_wanted = true;
+        return;
+    }
+    flush_wgrad(d);
+    Plan& p = *n.values_only;
+    n.values_only = nullptr;
+    NetArgsHost a = net_args(p);
+    float* kept = p.kept;
+    a.X = kept;
+    kept += p.columns() * n.neurons[0];
+    for (int t = 0; t + 2 < n.layers; ++t) {
+        if (n.weights_kept) a.W[t] = kept;
+        kept += n.param_count(t);
+    }
+    a.Z[n.layers - 1] = kept;  // the outputs in the arena stay as they are
+    if (n.split) refresh_operands(n, a.W);
+    n.ws_current = false;  // maybe those of kept weights (fp32 products: written by the forward)
+    int width = p.width;
+    void* args[] = {&a, &width};
+    TraceScope trace(d, kTraceNetworkForward, 0.0);
+    launch_module(d, p.fused->network_forward, unsigned(epoch_blocks(p)), 1, args, unsigned(p.fused->net_threads));
 }
 
 static void fused_forward(Plan& p) {
@@ -623,11 +673,16 @@ static void fused_forward(Plan& p) {
         // layers' stacks, which are most of such a forward's bytes (65,536 points
         // 2->128^4->1 83 -> 54 us; 10 rows of 32,768 points 3->128^5->1 470 -> 293).
         // (A recording writes every stack: their pointers may go out after it.)
-        const bool values = !p.backward && !n.stacks_out && !n.bound && !d.capturing;
+        const bool values = p.kept && !n.stacks_out && !n.bound && !d.capturing;
+        // where the weights' pointer is out, they may change at any time
+        if (values) a.keep = n.weights_out;
         launch_module(d, values ? fm.network_values : fm.network_forward,
                       unsigned((width + fm.net_points_per_block - 1) / fm.net_points_per_block), 1, args,
                       unsigned(fm.net_threads));
-        if (values) n.values_only = &p;
+        if (values) {
+            n.values_only = &p;
+            n.weights_kept = n.weights_out;
+        }
         if (!values) n.ws_current = true;  // fp32 products: written by the forward's side job
         return;
     }
@@ -693,7 +748,6 @@ static int wgrad_blocks_per_cu() { return std::max(1, env_int("CPDE_WGRAD_OCC", 
 // 0.0936/0.0954, 0.1033/0.1050; the Poisson graph epoch 0.0924 against 0.0943.
 static int wgrad_direct_blocks_per_cu() { return std::max(1, env_int("CPDE_WGRAD_DIRECT_OCC", 1)); }
 
-static int epoch_blocks(const Plan& p);
 static bool one_pass_fits(const Plan& p);
 
 // Cost records of a one-pass epoch of `blocks` workgroups (more than
@@ -1565,6 +1619,7 @@ int cpde_net_state(cpde_net* net, int transition, int buffer, float** device_ptr
         flush_reduce(*net->dev);
         require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
         if (buffer == 0) {  // the caller may write the weights
+            keep_weights(*net);
             net->ws_current = false;
             net->weights_out = true;
         }
@@ -1624,6 +1679,11 @@ int cpde_plan_create(cpde_net* net, int rows, int variables, const int* table, i
         if (fused_eligible(*net, *p)) {
             p->fused = load_fused(*net->dev, p->tables, net->neurons, width);
             p->network = network_mode();
+            if (p->network && !p->backward) {
+                size_t floats = p->columns() * (net->neurons[0] + net->neurons.back());
+                for (int t = 0; t + 2 < net->layers; ++t) floats += net->param_count(t);
+                HIP_CHECK(hipMalloc(&p->kept, floats * sizeof(float)));
+            }
         } else if (p->rows <= kRowsModuleRows && env_int("CPDE_FUSED", 1) && has_sigmoid(*net)) {
             p->rows_module = load_rows(*net->dev, p->tables);
         }
@@ -1638,6 +1698,7 @@ int cpde_plan_destroy(cpde_plan* plan) {
         Net& n = *plan->net;
         sync_stream(*n.dev, __LINE__);
         if (n.values_only == plan) n.values_only = nullptr;
+        (void)hipFree(plan->kept);
         if (n.bound && n.bound->plan == plan) {
             swap_binding(n, *plan, *n.bound);
             n.bound = nullptr;
@@ -1729,7 +1790,7 @@ int cpde_plan_stack(cpde_plan* plan, int layer, int kind, float** device_ptr) {
         require(p != nullptr, "stack not present for this layer");
         if (layer > 0 && layer + 1 < n.layers) {
             n.stacks_out = true;
-            if (n.values_only == plan && !n.dev->capturing) fused_forward(*plan);  // the stacks it left out
+            settle_arena(n);
         }
         *device_ptr = p;
     });
@@ -1759,7 +1820,6 @@ int cpde_activate(cpde_plan* plan, const float* data, int data_width, const int*
         require(valid >= 0 && valid <= plan->width && offset >= 0 && offset + valid <= data_width,
                 "invalid chunk range");
         reserve_arena(n, *plan);
-        if (n.values_only == plan) n.values_only = nullptr;  // its input is another now
         launch_activate(d, plan->input, data, data_width, n.neurons[0], plan_rows(*plan, rows), plan->rows, plan->width,
                         offset, valid);
     });
@@ -1935,6 +1995,7 @@ int cpde_backward(cpde_plan* plan, int accumulate) {
         Net& n = *plan->net;
         Device& d = *n.dev;
         require(plan->backward, "plan has no adjoint storage");
+        settle_arena(n);
         if (plan->fused) {
             fused_backward(*plan, accumulate != 0);
             return;
@@ -2371,6 +2432,7 @@ int cpde_capture_begin(cpde_device* dev) {
         require(!dev->tracing, "tracing times every launch with events; a capture cannot hold them");
         flush_reduce(*dev);
         dev->capture_nets.clear();
+        for (Net* n : dev->nets) n->arena_wanted = false;
         for (Net* n : dev->nets) dev->capture_nets.push_back({n, n->active, n->forwards, n->values_only});
         dev->capture_layout = dev->layout;
         HIP_CHECK(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
@@ -2386,6 +2448,8 @@ static void abandon_capture(Device& d) {
         c.net->active = c.active;
         c.net->ws_current = false;
         c.net->values_only = c.values_only;
+        if (c.net->arena_wanted) settle_arena(*c.net);
+        keep_weights(*c.net);
     }
     d.capture_nets.clear();
 }
@@ -2419,7 +2483,16 @@ int cpde_capture_end(cpde_device* dev, int keep, cpde_replay** out) {
         r->exec = exec;
         r->layout = dev->layout;
         for (auto& c : dev->capture_nets)
-            r->nets.push_back({c.net, c.active, c.net->active, c.net->generation, c.net->forwards != c.forwards});
+            r->nets.push_back({c.net, c.active, c.net->active, c.net->generation, c.net->forwards != c.forwards,
+                               c.net->arena_wanted});
+        for (auto& c : dev->capture_nets) {
+            if (c.net->arena_wanted) {
+                c.net->values_only = c.values_only;
+                settle_arena(*c.net);
+                refresh_operands(*c.net);
+            }
+            keep_weights(*c.net);
+        }
         // the recorded calls have done their host bookkeeping: their device
         // work runs now
         const hipError_t launched = hipGraphLaunch(exec, dev->stream);
@@ -2444,8 +2517,11 @@ int cpde_replay_launch(cpde_replay* replay) {
             require(c.net->generation == c.generation, "a network's stack arena changed since the capture");
         }
         flush_reduce(d);
-        for (const auto& c : replay->nets)
+        for (const auto& c : replay->nets) {
+            if (c.wanted) settle_arena(*c.net);
+            if (!c.forward) keep_weights(*c.net);
             if (!c.net->ws_current) refresh_operands(*c.net);
+        }
         HIP_CHECK(hipGraphLaunch(replay->exec, d.stream));
         for (const auto& c : replay->nets) {
             c.net->active = c.after;

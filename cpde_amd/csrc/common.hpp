@@ -124,9 +124,13 @@ struct Net {
     // without a backward write every stack, and so do one-pass epochs over more
     // workgroups than fit on the device together
     bool stacks_out = false;
-    // the plan whose forward ran last on the arena, where it wrote no stacks,
-    // and the forwards that ran there (the recorded ones as they are recorded)
-    const struct Plan* values_only = nullptr;
+    // the plan whose forward ran last on the arena, where it wrote no stacks
+    // (settle_arena writes them from its inputs and weights), and whether its
+    // weights are copied yet (Plan::kept); the forwards that ran there (recorded
+    // ones as they are recorded); and whether the stacks were wanted during the
+    // open capture
+    struct Plan* values_only = nullptr;
+    bool weights_kept = false, arena_wanted = false;
     uint64_t forwards = 0;
     // split-K partial buffer for the weight-gradient contraction
     float* partials = nullptr;
@@ -159,6 +163,10 @@ struct Plan {
     // the plan's activated chunk [point][row][channel] (layer 0): its own, so
     // that plans of one network keep their inputs between epochs
     float* input = nullptr;
+    // without a backward, on the network-fused kernels: the inputs and (once they
+    // may change) the weights of all but the output transition, as of the last
+    // forward that wrote no stacks, then room for outputs
+    float* kept = nullptr;
     std::shared_ptr<FusedModule> fused;  // null: one launch per product and composition
     std::shared_ptr<RowsModule> rows_module;  // their compositions (null: table-driven)
     bool network = false;                // fused: one network-wide kernel per pass
@@ -336,7 +344,7 @@ struct Device {
         Net* net;
         std::vector<int> active;
         uint64_t forwards;
-        const Plan* values_only;
+        Plan* values_only;
     };
     std::vector<NetCapture> capture_nets;  // state when the open capture began
     // Deferred gradient reductions (cpde_gradients_defer): a backward pass's
@@ -495,6 +503,9 @@ struct ScalarPublish {
 };
 // test: the launch tests the gradients for finiteness itself and writes the
 // gradient totals in their short form (only where update_tests(net) holds).
+// The weights are about to change: a copy for the stacks that the arena's last
+// forward left out.
+void keep_weights(Net& net);
 void launch_rprop(Device& d, Net& net, const UpdateGuard* guard = nullptr, const ScalarPublish* publish = nullptr,
                   bool test = false);
 // Adam step `step`; with `guard`, only where the rule accepts the epoch.

@@ -893,15 +893,26 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
         fwd << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L) << ">(a, " << t
             << ", X, T, p0, npts);\n";
     fwd << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
-    // the forward of a plan without a backward: outputs alone, no layer's stacks
+    // the forward of a plan without a backward: outputs alone, no layer's stacks,
+    // and a copy of the inputs and weights of those
     std::ostringstream val;
     val << "    const int p0 = net_block(a) * kNPB, npts = kNPB == 1 ? 1 : min(kNPB, points - p0);\n"
+        << "    const float xin = input_ahead<" << neurons[0] << ">(a, p0, npts);\n"
         << "    net_input<" << neurons[0] << ", " << neurons[1] << ", " << operand(L > 3) << ", false>(a, X, p0, npts);\n"
+        << "    net_keep_input<" << neurons[0] << ">(a, p0, npts, xin);\n"
         << "    __syncthreads();\n";
     for (int t = 1; t + 2 < L; ++t)
         val << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
             << ", kDropped, false>(a, " << t << ", X, T, p0, npts);\n";
     val << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
+    val << "    if (a.keep) {\n";
+    for (int t = 0, offset = 0; t + 2 < L; ++t) {
+        const int count = neurons[t + 1] * (neurons[t] + 1);
+        val << "        net_keep_weights<" << count << ">(a, " << t << ", size_t(points) * R * " << neurons[0] << " + "
+            << offset << ");\n";
+        offset += count;
+    }
+    val << "    }\n";
     {
         const std::string last = std::to_string(neurons[L - 2]);
         bwd << "    UAhead<" << last << ", output_adjoint_split<" << last << ">()> ua;\n    u_ahead<" << last

@@ -1619,6 +1619,7 @@ static unsigned reduce_grid(const ReduceArgs& a) {
 // transitions: transitions [first, first + a.transitions) of `net`, whose
 // active gradient buffers are a.grad.
 void launch_reduce_rprop(Device& d, const ReduceArgs& a, Net& net, int first) {
+    keep_weights(net);
     OptimizerArgs o{};
     o.transitions = a.transitions;
     o.split = net.split;
@@ -2369,6 +2370,7 @@ static void set_test(Device& d, OptimizerArgs& a, bool test) {
 }
 
 void launch_rprop(Device& d, Net& net, const UpdateGuard* guard, const ScalarPublish* publish, bool test) {
+    keep_weights(net);
     bool first = true;
     for_transition_groups(net, [&](OptimizerArgs a, int blocks) {
         if (guard) {
@@ -2389,6 +2391,7 @@ void launch_rprop(Device& d, Net& net, const UpdateGuard* guard, const ScalarPub
 
 void launch_adam(Device& d, Net& net, int step, float lr, const UpdateGuard* guard, const ScalarPublish* publish,
                  bool test) {
+    keep_weights(net);
     const float b1 = 0.9f, b2 = 0.999f;
     const float b1t = std::pow(b1, float(step)), b2t = std::pow(b2, float(step));
     bool first = true;

@@ -161,9 +161,9 @@ int cpde_activate(cpde_plan* plan, const float* data, int data_width, const int*
 /* network::feedforward (cuda/cpde_engine.cuh:889-913): every layer's linear step
  * (fp32 accuracy on MFMA, bias on the value row) and sigmoid composition through
  * order 6.  A plan without a backward writes its output stack alone on the
- * network-fused kernels; the layers' stacks follow (of the weights as they are
- * then) when cpde_plan_stack first asks for one, and with every forward from
- * then on. */
+ * network-fused kernels; the layers' stacks follow, as of that forward,
+ * when cpde_plan_stack first asks for one on the network, and with every
+ * forward from then on. */
 int cpde_forward(cpde_plan* plan);
 /* Copy the output stack's valid lanes to wire layout dest [dest_rows][dest_width][n_out]
  * (device), plan row r going to dest row rows[r] (Server::evaluate :171-183). */

@@ -9,7 +9,7 @@ from test_gpu_rows import workload
 
 pytestmark = pytest.mark.gpu
 
-POINTS = 9001   # more workgroups than CUs at every width here
+POINTS = 9001
 
 
 class Values:
@@ -123,3 +123,114 @@ def test_stacks_after_a_discarded_recording(device, neurons):
     device.capture_end(keep=False)
     same(v.stacks(), want)
     v.close()
+
+
+@pytest.mark.parametrize('order', [1, 6])   # several points per workgroup, one
+@pytest.mark.parametrize('held', [False, True])
+@pytest.mark.parametrize('neurons', WIDTHS + [[2, 130, 1]])
+def test_stacks_are_those_of_the_forward(device, neurons, held, order):
+    """Other weights and another chunk in the meantime, through the weights'
+    pointer of before the forward (held) or of after it; the outputs stay."""
+    want, outputs = expected(device, neurons, 0.25, order=order)
+    v = Values(device, neurons, order)
+    pointers = [v.net.state_ptr(t, 0)[0] for t in range(len(neurons) - 1)] if held else None
+    v.forward(0.25)
+    for t, w in enumerate(v.wl.init):
+        device.upload_ptr(pointers[t] if held else v.net.state_ptr(t, 0)[0], np.float32(0.5) * w)
+    device.upload_ptr(v.data.ptr, v.stack(0.5))
+    v.activate()
+    same(v.stacks(), want)
+    same([v.output()], [outputs])
+    for t, w in enumerate(v.wl.init):
+        v.net.set_state(t, 0, w)
+    v.plan.forward()   # the chunk that was activated, every stack
+    same(v.stacks(), expected(device, neurons, 0.5, order=order)[0])
+    v.close()
+
+
+@pytest.mark.parametrize('neurons', WIDTHS)
+def test_stacks_after_an_update(device, neurons):
+    """An RPROP update and an Adam update behind a forward, and weights of the
+    updated network in the next one."""
+    want, outputs = expected(device, neurons, 0.25)
+    runs = []
+    for backward in (False, True):
+        v = Values(device, neurons, backward=backward)
+        for t in range(len(neurons) - 1):
+            v.net.set_state(t, v.net.active(t), np.ones_like(v.wl.init[t]))
+        v.forward(0.25)
+        v.net.rprop()
+        v.net.adam(1, 1e-2)
+        if not backward:
+            same(v.stacks(), want)
+            same([v.output()], [outputs])
+        runs.append([v.forward().output()] + v.stacks())
+        v.close()
+    same(*runs)
+
+
+@pytest.mark.parametrize('neurons', WIDTHS)
+def test_bound_sets_and_the_arena_keep_their_own(device, neurons):
+    """A forward into a bound set, one in the arena before and after: each place
+    holds its own forward's stacks."""
+    in_set, set_outputs = expected(device, neurons, 0.25)
+    in_arena, outputs = expected(device, neurons, 0.5)
+    v = Values(device, neurons)
+    kept = hip.vp()
+    hip.check(hip.load().cpde_stacks_create(v.plan.handle, hip.ctypes.byref(kept)))
+    bind = hip.load().cpde_plan_bind
+    v.forward(0.5)
+    hip.check(bind(v.plan.handle, kept))
+    v.forward(0.25)
+    for t, w in enumerate(v.wl.init):
+        v.net.set_state(t, 0, 0.5 * w)
+    same(v.stacks(), in_set)
+    same([v.output()], [set_outputs])
+    hip.check(bind(v.plan.handle, None))
+    same(v.stacks(), in_arena)
+    same([v.output()], [outputs])
+    hip.check(bind(v.plan.handle, kept))
+    same(v.stacks(), in_set)
+    hip.check(bind(v.plan.handle, None))
+    hip.check(hip.load().cpde_stacks_destroy(kept))
+    v.close()
+
+
+@pytest.mark.parametrize('neurons', WIDTHS)
+@pytest.mark.parametrize('keep', [True, False])
+def test_stacks_asked_for_inside_a_capture(device, neurons, keep):
+    """Of a forward before the capture, in a recording that runs none."""
+    want, outputs = expected(device, neurons, 0.25)
+    v = Values(device, neurons)
+    v.forward(0.25)
+    v.output()   # its rows are on the device before the capture
+    device.capture_begin()
+    pointer = v.plan.stack_ptr(1, 1)
+    v.plan.output(v.out, POINTS, v.rows, 0, POINTS)
+    replay = device.capture_end(keep)
+    got = device.download_ptr(pointer, np.float32, want[0].size).reshape(want[0].shape)
+    same([got] + v.stacks(), [want[0]] + want)
+    same([v.output()], [outputs])
+    if replay:
+        replay.launch()
+        same(v.stacks(), want)
+        replay.destroy()
+    v.close()
+
+
+def test_backward_of_another_plan_reads_the_arena(device):
+    """A backward plan's adjoints of a forward that another plan ran."""
+    neurons = [2, 40, 24, 1]
+    adjoint = np.random.default_rng(3).standard_normal((POINTS, 3, 1)).astype(np.float32)
+    got = []
+    for plain in (False, True):
+        v = Values(device, neurons)
+        other = Values(device, neurons, net=v.net, backward=True)
+        other.activate()
+        (other if plain else v).forward(0.0)
+        device.upload_ptr(other.plan.stack_ptr(3, 2), adjoint)
+        other.plan.backward()
+        got.append([v.net.gradient(t) for t in range(3)])
+        other.close()
+        v.close()
+    same(*got)
