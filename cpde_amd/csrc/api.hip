@@ -1628,6 +1628,34 @@ int cpde_net_state(cpde_net* net, int transition, int buffer, float** device_ptr
     });
 }
 
+int cpde_net_read(cpde_net* net, int transition, int buffer, float* values) {
+    return guarded([&] {
+        Device& d = *net->dev;
+        flush_reduce(d);
+        require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
+        require(values != nullptr, "null argument");
+        HIP_CHECK(hipMemcpyAsync(values, net->state[buffer][transition], net->param_count(transition) * sizeof(float),
+                                 hipMemcpyDeviceToHost, d.stream));
+        sync_stream(d, __LINE__);
+    });
+}
+
+int cpde_net_write(cpde_net* net, int transition, int buffer, const float* values) {
+    return guarded([&] {
+        Device& d = *net->dev;
+        flush_reduce(d);
+        require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
+        require(values != nullptr, "null argument");
+        if (buffer == 0) {
+            keep_weights(*net);
+            net->ws_current = false;
+        }
+        HIP_CHECK(hipMemcpyAsync(net->state[buffer][transition], values, net->param_count(transition) * sizeof(float),
+                                 hipMemcpyHostToDevice, d.stream));
+        sync_stream(d, __LINE__);
+    });
+}
+
 int cpde_net_active(cpde_net* net, int transition) {
     if (!net || transition < 0 || transition >= net->layers - 1) return -1;
     return net->active[transition];

@@ -2185,6 +2185,7 @@ __global__ __launch_bounds__(256) void weight_operand_kernel(WeightOperandArgs a
 void launch_weight_operands(Device& d, const float* const* W, void* const* WS, const int* n_in, const int* n_out,
                             int count, bool split) {
     for (int first = 0; first < count; first += kMaxTransitions) {
+        TraceScope trace(d, kTraceOther, 0.0);
         WeightOperandArgs a{};
         a.split = split;
         a.transitions = std::min(kMaxTransitions, count - first);

@@ -1222,11 +1222,8 @@ Frame Server::snapshot(NetRecord& n) {
     for (int t = 0; t < n.transitions(); ++t) {
         b.put<int32_t>(cpde_net_active(n.net, t));
         for (int k = 0; k < 4; ++k) {
-            float* ptr = nullptr;
-            int count = 0;
-            call(cpde_net_state(n.net, t, k, &ptr, &count));
-            std::vector<float> v(count);
-            call(cpde_buffer_download(dev_, v.data(), ptr, v.size() * sizeof(float)));
+            std::vector<float> v(size_t(n.neurons[t + 1]) * (n.neurons[t] + 1));
+            call(cpde_net_read(n.net, t, k, v.data()));
             b.put_array(v);
         }
     }
@@ -1259,13 +1256,7 @@ void Server::restore(NetRecord& n, Frame& b) {
     call(cpde_device_synchronize(dev_));
     for (int t = 0; t < n.transitions(); ++t) {
         call(cpde_net_set_active(n.net, t, active[t]));
-        for (int k = 0; k < 4; ++k) {
-            float* ptr = nullptr;
-            int count = 0;
-            call(cpde_net_state(n.net, t, k, &ptr, &count));
-            const auto& v = arrays[size_t(t) * 4 + k];
-            call(cpde_buffer_upload(dev_, ptr, v.data(), v.size() * sizeof(float)));
-        }
+        for (int k = 0; k < 4; ++k) call(cpde_net_write(n.net, t, k, arrays[size_t(t) * 4 + k].data()));
     }
     n.optimizer = optimizer;
     n.updates = updates;

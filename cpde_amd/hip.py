@@ -50,6 +50,8 @@ SIGNATURES = {
     'cpde_buffer_copy': (i32, [vp, vp, vp, ctypes.c_size_t]),
     'cpde_net_create': (i32, [vp, i32, vp, vp, vp, ctypes.POINTER(vp)]),
     'cpde_net_destroy': (i32, [vp]),
+    'cpde_net_read': (i32, [vp, i32, i32, vp]),
+    'cpde_net_write': (i32, [vp, i32, i32, vp]),
     'cpde_net_state': (i32, [vp, i32, i32, ctypes.POINTER(vp), ctypes.POINTER(i32)]),
     'cpde_net_active': (i32, [vp, i32]),
     'cpde_net_set_active': (i32, [vp, i32, i32]),
@@ -277,15 +279,19 @@ class Net:
         check(load().cpde_net_state(self.handle, t, b, ctypes.byref(p), ctypes.byref(c)))
         return p, c.value
 
+    def _count(self, t):
+        assert 0 <= t < len(self.neurons) - 1
+        return self.neurons[t + 1] * (self.neurons[t] + 1)
+
     def state(self, t, b):
-        p, c = self.state_ptr(t, b)
-        return self.device.download_ptr(p, np.float32, c)
+        v = np.empty(self._count(t), np.float32)
+        check(load().cpde_net_read(self.handle, t, b, _ptr(v)))
+        return v
 
     def set_state(self, t, b, values):
-        p, c = self.state_ptr(t, b)
         v = np.ascontiguousarray(values, np.float32)
-        assert v.size == c
-        self.device.upload_ptr(p, v)
+        assert v.size == self._count(t)
+        check(load().cpde_net_write(self.handle, t, b, _ptr(v)))
 
     def active(self, t):
         return load().cpde_net_active(self.handle, t)

@@ -110,6 +110,12 @@ int cpde_net_destroy(cpde_net* net);
  * after writing (the library keeps a copy of the weights as its products'
  * operands, which it rebuilds after the pointer has been handed out). */
 int cpde_net_state(cpde_net* net, int transition, int buffer, float** device_ptr, int* count);
+/* Copy a whole state buffer to or from host memory (synchronous).  No pointer
+ * goes out, so the library knows when the weights change: a network whose
+ * weights' pointer is out has its products' operands rebuilt by every separate
+ * forward. */
+int cpde_net_read(cpde_net* net, int transition, int buffer, float* values);
+int cpde_net_write(cpde_net* net, int transition, int buffer, const float* values);
 /* The active gradient buffer (1 or 2) of a transition (weights::act_grad). */
 int cpde_net_active(cpde_net* net, int transition);
 int cpde_net_set_active(cpde_net* net, int transition, int active);
