@@ -26,6 +26,7 @@ struct cpde_replay_s {
         // whether it runs a forward on the network's arena, and whether stacks of
         // an earlier one were wanted while it was recorded
         bool forward, wanted;
+        bool separate;  // whether it runs a separate forward
     };
     std::vector<NetState> nets;
 };
@@ -664,6 +665,7 @@ static void fused_forward(Plan& p) {
     const double cols = double(p.columns());
     if (p.network) {
         if (n.split && (!n.ws_current || n.weights_out)) refresh_operands(n);
+        n.separate = true;
         NetArgsHost a = net_args(p);
         void* args[] = {&a, &width};
         double flops = 0;
@@ -2460,7 +2462,7 @@ int cpde_capture_begin(cpde_device* dev) {
         require(!dev->tracing, "tracing times every launch with events; a capture cannot hold them");
         flush_reduce(*dev);
         dev->capture_nets.clear();
-        for (Net* n : dev->nets) n->arena_wanted = false;
+        for (Net* n : dev->nets) n->arena_wanted = n->separate = false;
         for (Net* n : dev->nets) dev->capture_nets.push_back({n, n->active, n->forwards, n->values_only});
         dev->capture_layout = dev->layout;
         HIP_CHECK(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
@@ -2512,7 +2514,7 @@ int cpde_capture_end(cpde_device* dev, int keep, cpde_replay** out) {
         r->layout = dev->layout;
         for (auto& c : dev->capture_nets)
             r->nets.push_back({c.net, c.active, c.net->active, c.net->generation, c.net->forwards != c.forwards,
-                               c.net->arena_wanted});
+                               c.net->arena_wanted, c.net->separate});
         for (auto& c : dev->capture_nets) {
             if (c.net->arena_wanted) {
                 c.net->values_only = c.values_only;
@@ -2548,7 +2550,8 @@ int cpde_replay_launch(cpde_replay* replay) {
         for (const auto& c : replay->nets) {
             if (c.wanted) settle_arena(*c.net);
             if (!c.forward) keep_weights(*c.net);
-            if (!c.net->ws_current) refresh_operands(*c.net);
+            // (as before a separate forward: the pointer's holder may have written again)
+            if (!c.net->ws_current || (c.net->split && c.separate && c.net->weights_out)) refresh_operands(*c.net);
         }
         HIP_CHECK(hipGraphLaunch(replay->exec, d.stream));
         for (const auto& c : replay->nets) {

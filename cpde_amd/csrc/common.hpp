@@ -115,6 +115,7 @@ struct Net {
     // write again.
     std::vector<void*> ws;
     bool split = false, ws_current = false, weights_out = false;
+    bool separate = false;  // the open capture holds a separate forward
     // Stack arena shared by every plan of the network (contexts are views,
     // the reference's layer banks, cuda/cpde_engine.cuh:661-693).
     std::vector<float*> z, y, g;      // per layer

@@ -63,3 +63,38 @@ def test_operands_are_rebuilt_after_a_write_alone(device):
             assert call(f.handle, *bad, v.ctypes.data) == hip.EINVAL
         f.destroy()
 
+
+@pytest.mark.parametrize('width', [128, 40])
+def test_replayed_forwards_see_weights_written_through_a_held_pointer(device, width):
+    f = Forward(device, [2, width, width, 1])
+    first = f.outputs()
+    pointer, count = f.net.state_ptr(1, 0)
+    f.run()
+    device.capture_begin()
+    f.run()
+    replay = device.capture_end()
+    for _ in range(2):
+        device.upload_ptr(pointer, np.zeros(count, np.float32))
+        replay.launch()
+        assert not np.array_equal(f.outputs(), first)
+        device.upload_ptr(pointer, np.ascontiguousarray(f.wl.init[1], np.float32))
+        replay.launch()
+        assert np.array_equal(f.outputs(), first)
+    replay.destroy()
+
+    # recorded before the pointer went out
+    g = Forward(device, [2, width, width, 1])
+    device.capture_begin()
+    g.run()
+    replay = device.capture_end()
+    pointer, count = g.net.state_ptr(1, 0)
+    for _ in range(2):
+        device.upload_ptr(pointer, np.zeros(count, np.float32))
+        replay.launch()
+        assert not np.array_equal(g.outputs(), first)
+        device.upload_ptr(pointer, np.ascontiguousarray(f.wl.init[1], np.float32))
+        replay.launch()
+        assert np.array_equal(g.outputs(), first)
+    replay.destroy()
+    f.close()
+    g.close()
