@@ -826,7 +826,8 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
         // direct tiles everywhere.
         for (int k = 0; k < T; ++k) {
             const int M = n.neurons[first + k + 1], N = n.neurons[first + k];
-            if (external_splits[first + k] || !wide(k)) continue;
+            // (few columns are short sums, as in launch_gemm)
+            if (external_splits[first + k] || !wide(k) || K <= kShortSum) continue;
             split = true;
             has256 = has256 || std::max(M, N) > 128;
         }

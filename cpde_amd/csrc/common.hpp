@@ -457,6 +457,7 @@ void launch_output(Device& d, float* dest, const float* out, int dest_width, int
                    int rows, int width, int offset, int valid);
 void launch_compose_forward(Device& d, const Plan& p, const float* z, float* y, int n);
 void launch_compose_adjoint(Device& d, const Plan& p, const float* z, float* g, int n);
+constexpr int kShortSum = 3;  // terms up to which a product stays on fp32 instructions
 // C[M x N] = A[M x K] B[N x K]^T: B k-contiguous (B[k + ldb*n]), A k-contiguous
 // (a_k: A[k + lda*m]) or m-contiguous (A[m + lda*k]), C[m + ldc*n].  bias (may be
 // null) is added to every column n with n % period == 0.

@@ -551,6 +551,7 @@ __device__ __forceinline__ float upper_half(float x) { return __uint_as_float(__
 
 // Eight values into their three planes.
 __device__ __forceinline__ void split_planes(const float (&x)[8], uintx4 (&plane)[3]) {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float a = x[2 * i], b = x[2 * i + 1];
@@ -841,10 +842,64 @@ static void split_gemm(Device& d, int M, int N, int K, const float* A, int lda, 
     run(d, M, N, K, A, lda, B, ldb, C, ldc, bias, period);
 }
 
+// The same for sums of up to kShortSum terms, on fp32 vector instructions: the
+// three products that a split leaves out (2^-26 of a term in the mean, 2^-22.4
+// at most) show where there are no more terms for them to drown among (relative to
+// the terms' norm, rms and most, 200,000 sums: one term 3.4e-8 and 2.1e-7 split,
+// 2.5e-8 and 6.0e-8 here; three 3.4e-8 and 2.1e-7, 3.6e-8 and 1.8e-7; 128 terms
+// 3.4e-8 and 2.0e-7, 2.0e-7 and 1.6e-6).  A lane keeps V adjacent rows of A for
+// all of its columns.
+template <bool A_K, int V>
+__global__ __launch_bounds__(256) void short_gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
+                                                         const float* __restrict__ B, int ldb, float* __restrict__ C,
+                                                         int ldc, const float* __restrict__ bias, int period) {
+    typedef float rows __attribute__((ext_vector_type(V)));
+    const unsigned lane = blockIdx.x * 256 + threadIdx.x, groups = M / V, step = gridDim.x * 256 / groups;
+    unsigned n = lane / groups;
+    const unsigned m = (lane - n * groups) * V;
+    if (n >= step) return;
+    rows a[kShortSum], add;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        add[v] = bias ? bias[m + v] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < kShortSum; ++k)
+            a[k][v] = k >= K ? 0.0f : A_K ? A[k + size_t(lda) * (m + v)] : A[m + v + size_t(lda) * k];
+    }
+#pragma unroll 4
+    for (; n < unsigned(N); n += step) {
+        rows sum;
+#pragma unroll
+        for (int v = 0; v < V; ++v) sum[v] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kShortSum; ++k) {
+            const float b = k < K ? B[k + size_t(ldb) * n] : 0.0f;
+#pragma unroll
+            for (int v = 0; v < V; ++v) sum[v] = k < K ? fmaf(a[k][v], b, sum[v]) : sum[v];
+        }
+        if (bias && n % unsigned(period) == 0) sum += add;
+        *reinterpret_cast<rows*>(C + m + size_t(ldc) * n) = sum;
+    }
+}
+
+template <bool A_K>
+static void short_gemm(Device& d, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C,
+                       int ldc, const float* bias, int period) {
+    const int V = M % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 ? 4 : 1;
+    const size_t groups = M / V, blocks = std::min<size_t>((groups * N + 255) / 256, 8 * size_t(d.compute_units));
+    const auto kernel = V == 4 ? short_gemm_kernel<A_K, 4> : short_gemm_kernel<A_K, 1>;
+    hipLaunchKernelGGL(kernel, unsigned(std::max(blocks, (groups + 255) / 256)), 256, 0, d.stream, M, N, K, A, lda, B,
+                       ldb, C, ldc, bias, period);
+    HIP_CHECK(hipGetLastError());
+}
+
 void launch_gemm(Device& d, int M, int N, int K, const float* A, int lda, bool a_k, const float* B, int ldb, float* C,
                  int ldc, const float* bias, int period) {
     if (M <= 0 || N <= 0) return;
     TraceScope trace(d, a_k ? kTraceGemmTransposed : kTraceGemm, 2.0 * M * double(N) * K);
+    if (K <= kShortSum)
+        return (a_k ? short_gemm<true> : short_gemm<false>)(d, M, N, K, A, lda, B, ldb, C, ldc, bias,
+                                                            period > 0 ? period : 1);
     const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool vec = M % 4 == 0 && K % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && aligned(A) &&
                      aligned(B) && aligned(C) && aligned(bias);
@@ -999,6 +1054,7 @@ __device__ __forceinline__ bool update_applies(const OptimizerArgs& a, bool fini
 // plane, lane (q, j) and place in the lane's eight -- the forward's with m = o,
 // k = i, the backward's with m = i, k = o.
 __device__ __forceinline__ void weight_operand(unsigned short* ws, int n_in, int n_out, int o, int i, float w) {
+#pragma clang fp contract(off)
     const float r = w - upper_half(w);
     const unsigned mid = __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{r, r}, bf16x2));
     const unsigned short plane[3] = {static_cast<unsigned short>(__float_as_uint(w) >> 16),
