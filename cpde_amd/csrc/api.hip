@@ -777,73 +777,81 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     GradientPlan g;
     // local transition k is the network's transition first + k
     auto thin = [&](int k) { return n.neurons[first + k + 1] <= 16 || n.neurons[first + k] <= 16; };
-    // 128x128 tiles, or 64x64 when both widths are at most 64 -- or when the
-    // 128x128 splits would be short (fewer than kWgradMinColumns columns each):
-    // then four times the tiles give each split four times the columns, and
-    // the split partials the reduction reads shrink fourfold
-    bool small_tiles = false, direct = false, split = false, has256 = false;
-    auto wide = [&](int k) { return n.neurons[first + k + 1] > 64 && n.neurons[first + k] > 64; };
-    auto tile_of = [&](int k) {
-        if (split && wide(k)) return std::max(n.neurons[first + k + 1], n.neurons[first + k]) > 128 ? 256 : 128;
-        return direct || small_tiles || (n.neurons[first + k + 1] <= 64 && n.neurons[first + k] <= 64) ? 64 : 128;
+    auto widths = [&](int k) { return std::minmax(n.neurons[first + k + 1], n.neurons[first + k]); };
+    auto tiles_at = [&](int k, int tile) {
+        return ((n.neurons[first + k + 1] + tile - 1) / tile) * ((n.neurons[first + k] + tile - 1) / tile);
     };
-    auto tiles_of = [&](int k) {
-        const int T0 = tile_of(k);
-        return ((n.neurons[first + k + 1] + T0 - 1) / T0) * ((n.neurons[first + k] + T0 - 1) / T0);
-    };
-    auto count_tiles = [&] {
+    // The tile of every transition that the launch computes in tiles.  64x64 tiles
+    // fed straight from global memory, one per CU, beat the LDS-staged ones (128x128,
+    // 64x64 where both widths are at most 64 or where those splits would be short,
+    // fewer than kWgradMinColumns columns each) on long reductions too:
+    // 2->256^4->1 over 65,536-point chunks 25.9 -> 24.8 ms of weight gradient per
+    // epoch, 3->128^5->1 over 32,768 points 1.37 -> 1.27 ms.  CPDE_WGRAD_DIRECT=0
+    // keeps the LDS-staged tiles.
+    const bool staged = env_int("CPDE_WGRAD_DIRECT", -1) == 0;
+    std::vector<int> tile(T, 0);
+    auto count_tiles = [&](auto weight) {
         int total = 0;
         for (int k = 0; k < T; ++k)
-            if (!thin(k) && !external_splits[first + k]) total += tiles_of(k);
+            if (tile[k]) total += tiles_at(k, tile[k]) * weight(tile[k]);
         return total;
     };
-    // whole waves of tiles: a partial last wave would run alone for a whole split
-    auto splits_for = [&](int tiles) {
-        int per_cu = direct ? wgrad_direct_blocks_per_cu() : wgrad_blocks_per_cu();
-        // two split tiles of 128 share a CU where that leaves them long
-        if (split && !has256 && double(K) * tiles >= 2.0 * 2048 * d.compute_units) per_cu = 2;
-        return std::max(1, per_cu * d.compute_units / std::max(1, tiles));
+    auto one = [](int) { return 1; };
+    for (int k = 0; k < T; ++k)
+        if (!thin(k) && !external_splits[first + k]) tile[k] = staged && widths(k).second > 64 ? 128 : 64;
+    if (staged && K / std::max(1, wgrad_blocks_per_cu() * d.compute_units / std::max(1, count_tiles(one))) < kWgradMinColumns)
+        for (int& t : tile) t = t ? 64 : 0;
+    // Split tiles (bf16 matrix instructions at fp32 accuracy) for transitions wider
+    // than 64 on both sides; short sums (kShortSum) stay on direct tiles, and
+    // CPDE_WGRAD_SPLIT=0 keeps those everywhere.
+    //   256x256 tiles where a side is wider than 128, in a launch of their own with
+    // splits of their own: 2->256^4->1 over 65,536-point chunks 24.9 -> 15.8 ms of
+    // weight gradient per epoch (19.1 with 128x128 tiles, two per CU); 2->512^3->1 over
+    // 12,288 columns 160 -> 125 us.  They need the tile filled, by as many direct tiles
+    // as cost more: ten, eight where a width off 64 masks those (at order 6 over 8,192
+    // points, direct and split: 128->256 144 and 170 us, 384->384 652 and 733, 300->300
+    // 627 and 716; 512->300 1,053 and 758, 256->70 255 and 184, 200->200 333 and 180),
+    // and 256 columns a split, as a split's partials are 16 direct tiles' (512->512
+    // over 4,374 columns, 68 a split, 47 and 58 us; over 12,288, 192, 89 and 82;
+    // 384->384 over 12,288 59 and 72).
+    //   128x128 tiles otherwise, at 512 columns a split: 3->128^5->1 over 32,768
+    // points 1.32 -> 0.98 ms, the stacks' bytes at the rate of a copy; with 240
+    // (2->128^4->1, 20,412 columns) the direct tiles stay ahead, 22 against 27 us.
+    // Beside direct tiles in the launch one takes 2.5 times as long over a column,
+    // and as many more splits, and pays for masked widths alone (2->96^2->64->1 at order
+    // 6 over 8,192 points 167 -> 139 us, 2->128->64->128^2->1 174 -> 191).
+    auto cost = [&](int t) { return staged || t == 64 ? 2 : t == 128 ? 5 : 0; };  // in the launch of the smaller tiles
+    auto exact = [&](int k) { return widths(k).first % 64 == 0 && widths(k).second % 64 == 0; };
+    auto clear_split = [&](int size) {
+        for (int k = 0; k < T; ++k)
+            if (tile[k] == size) tile[k] = 64;
     };
-    int total_tiles = count_tiles();
-    // 64x64 tiles fed straight from global memory, one per CU.  They beat the
-    // LDS-staged tiles on long reductions too: 2->256^4->1 over 65,536-point
-    // chunks 25.9 -> 24.8 ms of weight gradient per epoch, 3->128^5->1 over
-    // 32,768 points 1.37 -> 1.27 ms.  CPDE_WGRAD_DIRECT=0 keeps the LDS-staged
-    // tiles (128x128, or 64x64 where those splits would be short).
-    const bool staged = env_int("CPDE_WGRAD_DIRECT", -1) == 0;
-    if (total_tiles > 0 && !staged) {
-        small_tiles = true;
-        direct = true;
-        // Split tiles (bf16 matrix instructions at fp32 accuracy) for transitions
-        // wider than 64 on both sides: 256x256 where a side is wider than 128,
-        // else 128x128 where a tile's split stays long.  2->256^4->1 over 65,536-point
-        // chunks 24.9 -> 15.8 ms of weight gradient per epoch (19.1 with 128x128
-        // tiles, two per CU); 3->128^5->1 over 32,768 points 1.32 -> 0.98 ms, the
-        // stacks' bytes at the rate of a copy; 2->512^3->1 over 12,288 columns 525 ->
-        // 98 us.  With 240 columns a split (2->128^4->1, 20,412 columns) the direct
-        // tiles stay ahead, 22 against 27 us: a split tile then writes four times the
-        // partials, and the reduction grows from 5 to 9 us.  CPDE_WGRAD_SPLIT=0 keeps the
-        // direct tiles everywhere.
+    if (!staged && K > kShortSum && env_int("CPDE_WGRAD_SPLIT", 1)) {
         for (int k = 0; k < T; ++k) {
-            const int M = n.neurons[first + k + 1], N = n.neurons[first + k];
-            // (few columns are short sums, as in launch_gemm)
-            if (external_splits[first + k] || !wide(k) || K <= kShortSum) continue;
-            split = true;
-            has256 = has256 || std::max(M, N) > 128;
+            if (!tile[k] || widths(k).first <= 64) continue;
+            if (widths(k).second <= 128) tile[k] = 128;
+            else if (tiles_at(k, 64) >= (exact(k) ? 10 : 8) * tiles_at(k, 256)) tile[k] = 256;
         }
-        if (split) total_tiles = count_tiles();
-        if (split && !has256 && double(K) * total_tiles < 512.0 * d.compute_units) split = false;
-        if (!env_int("CPDE_WGRAD_SPLIT", 1)) split = false;
-        total_tiles = count_tiles();
-    } else if (total_tiles > 0 && K / splits_for(total_tiles) < kWgradMinColumns) {
-        small_tiles = true;
-        total_tiles = count_tiles();
+        if (double(K) * count_tiles([](int t) { return t == 256; }) < 256.0 * d.compute_units) clear_split(256);
+        if (std::count(tile.begin(), tile.end(), 64))
+            for (int k = 0; k < T; ++k)
+                if (tile[k] == 128 && exact(k)) tile[k] = 64;
+        if (double(K) * count_tiles(cost) < 512.0 * 5 * d.compute_units) clear_split(128);
     }
+    auto has = [&](int size) { return !staged && std::count(tile.begin(), tile.end(), size) > 0; };
+    // whole waves of tiles: a partial last wave would run alone for a whole split
+    auto splits_for = [&](int t) {
+        if (t == 256) return std::max(1, d.compute_units / count_tiles([](int u) { return u == 256; }));
+        int per_cu = staged ? wgrad_blocks_per_cu() : wgrad_direct_blocks_per_cu();
+        // two split tiles of 128 share a CU where that leaves them long
+        if (has(128) && double(K) * count_tiles(cost) >= 2.0 * 2048 * 5 * d.compute_units) per_cu = 2;
+        return std::max(1, per_cu * d.compute_units * cost(t) / count_tiles(cost));
+    };
     // transition k's splits, each of *chunk columns
     auto splits_of = [&](int k, int* chunk) {
         int s = external_splits[first + k];
         if (s) return s;
-        s = thin(k) ? 2 * d.compute_units : splits_for(total_tiles);
+        s = thin(k) ? 2 * d.compute_units : splits_for(tile[k]);
         s = std::max(1, std::min(s, std::max(1, K / kWgradChunk)));
         *chunk = (K + s - 1) / s;
         *chunk = (*chunk + kWgradChunk - 1) / kWgradChunk * kWgradChunk;
@@ -852,16 +860,16 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     // A one-pass epoch gives the same bits with and without the static scratch,
     // so where the split tiles' partials do not fit it, every call of the plan
     // takes the direct tiles, whose partials are a sixteenth.
-    if (split && one_pass_fits(p)) {
+    if ((has(128) || has(256)) && one_pass_fits(p)) {
         size_t floats = 0;
         for (int k = 0, chunk; k < T; ++k)
             floats += size_t(splits_of(k, &chunk)) * n.neurons[first + k + 1] * (n.neurons[first + k] + 1);
         if (floats > static_partial_floats(epoch_blocks(p))) {
-            split = has256 = false;
-            total_tiles = count_tiles();
+            clear_split(256);
+            clear_split(128);
         }
     }
-    g.wa.direct = split ? 2 : direct ? 1 : 0;
+    g.wa.direct = has(128) || has(256) ? 2 : staged ? 0 : 1;
     g.wa.block_begin[0] = 0;
     g.ra.accumulate = accumulate ? 1 : 0;
     g.ra.transitions = T;
@@ -874,13 +882,13 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
         int chunk = 0;
         const int s = splits_of(k, &chunk);
         if (!external_splits[t]) {
-            const int tiles = thin(k) ? 1 : tiles_of(k);
+            const int tiles = thin(k) ? 1 : tiles_at(k, tile[k]);
             g.wa.M[w] = M;
             g.wa.N[w] = N;
             g.wa.K[w] = K;
             g.wa.R[w] = p.rows;
             g.wa.kchunk[w] = chunk;
-            g.wa.tile[w] = tile_of(k);
+            g.wa.tile[w] = tile[k];
             g.wa.block_begin[w + 1] = g.wa.block_begin[w] + tiles * s;
             g.wa.G[w] = n.g[t + 1];
             g.wa.Y[w] = activations(p, t);

@@ -1648,8 +1648,10 @@ void launch_wgrad_grouped(Device& d, const WgradArgs& a, double flops) {
         if (wide.transitions)
             hipLaunchKernelGGL(vec ? wgrad_split256_kernel<true> : wgrad_split256_kernel<false>,
                                wide.block_begin[wide.transitions], 512, 0, d.stream, wide);
+        const bool split = std::count(rest.tile, rest.tile + rest.transitions, 128) > 0;
         if (rest.transitions)
-            hipLaunchKernelGGL(wgrad_split_kernel, rest.block_begin[rest.transitions], 256, 0, d.stream, rest);
+            hipLaunchKernelGGL(split ? wgrad_split_kernel : wgrad_direct_kernel, rest.block_begin[rest.transitions], 256, 0,
+                               d.stream, rest);
     } else if (a.direct)
         hipLaunchKernelGGL(wgrad_direct_kernel, a.block_begin[a.transitions], 256, 0, d.stream, a);
     else
