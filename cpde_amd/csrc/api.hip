@@ -432,7 +432,8 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     t.scaled = env_int("CPDE_SCALED", t.scaled) ? 1 : 0;
     // Wave priorities by dispatch round (tier_raise in the generated source).
     const int blocks = (width + t.net_points_per_block - 1) / t.net_points_per_block;
-    if (env_int("CPDE_NET_TIERS", 1) && widest < 128 && blocks > compute_units && resident(blocks, compute_units))
+    if (env_int("CPDE_NET_TIERS", 1) && !split_products(neurons) && blocks > compute_units &&
+        resident(blocks, compute_units))
         t.tier_cus = compute_units;
     t.keep_asked = one_pass_any_length(neurons) && !resident(blocks, compute_units);
     // Diagnostics: clock stamps of the one-pass epoch's phases, written over

@@ -686,9 +686,28 @@ static int forward_split_cap(const Tables& t, const FusedTuning& tuning) {
 }
 
 // Whether a network's products run on split bf16 operands (fused.hip.in); a
-// single hidden layer has none.
+// single hidden layer has none.  They pay from 128 neurons on, but the operand
+// planes are as wide as the widest layer, half as large again as fp32 ones, and
+// leave a CU fewer workgroups.  Where the other layers' products are small beside
+// that the fp32 ones are as fast on short grids and faster on long ones, at widths
+// that fill their tiles (ms per epoch at order 6 over 8,192 points, order 2 over
+// 16,384, split and fp32): 256->64 0.632 and 0.501, 0.302 and 0.257; 256^2->64 1.50
+// and 1.36, 0.708 and 0.644; 256->128 0.674 and 0.684, 0.396 and 0.370; 256->192
+// 0.845 and 0.892, 0.487 and 0.497; 128->96 0.328 and 0.345, 0.158 and 0.164;
+// 128->100, which masks fp32 tiles, 0.382 and 0.395, 0.162 and 0.182; 250->20^2,
+// with next to no products, 0.787 and 0.661, 0.337 and 0.306.
 bool split_products(const std::vector<int>& neurons) {
-    return neurons.size() > 3 && *std::max_element(neurons.begin() + 1, neurons.end() - 1) >= 128;
+    if (neurons.size() <= 3) return false;
+    int widest = 0, narrowest = neurons[1], total = 0, products = 0;
+    bool whole = true;  // 16-column tiles
+    for (size_t l = 1; l + 1 < neurons.size(); ++l) {
+        widest = std::max(widest, neurons[l]);
+        narrowest = std::min(narrowest, neurons[l]);
+        total += neurons[l];
+        if (l > 1) products += neurons[l - 1] * neurons[l];
+        whole = whole && neurons[l] % 16 == 0;
+    }
+    return widest >= 128 && 8.0 * products >= double(widest) * total && !(whole && 2 * narrowest <= widest);
 }
 
 namespace {

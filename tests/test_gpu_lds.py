@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize('variables,order,neurons,points', [
     (2, 6, [2, 80, 256, 1], 4133),
+    (2, 6, [2, 128, 240, 1], 4133),
     (3, 5, [3, 256, 1], 4101),
 ])
 def test_two_points_in_one_tile(device, variables, order, neurons, points):

@@ -89,12 +89,12 @@ def test_network_products(device, neurons):
 
 @pytest.mark.parametrize('narrow', [1, 2, 3])
 def test_short_network_products(device, narrow):
-    n = Layers(device, [1, 128, narrow, 130, 1], 1, 700)
-    z, _, total = n.product(2, n.stack(2, 1))
-    u, y = n.stack(3, 3)[:, 0], n.stack(3, 1)[:, 1]
+    n = Layers(device, [1, 128, 128, narrow, 130, 1], 1, 700)
+    z, _, total = n.product(3, n.stack(3, 1))
+    u, y = n.stack(4, 3)[:, 0], n.stack(4, 1)[:, 1]
     check('forward', (y - u * z[:, 1]) / (u * total[:, 1]), most=narrow + 1.0)
-    g, _, total = n.product(1, n.stack(2, 2), transposed=True)
-    u, got = n.stack(1, 3)[:, 0], n.stack(1, 2)[:, 1]
+    g, _, total = n.product(2, n.stack(3, 2), transposed=True)
+    u, got = n.stack(2, 3)[:, 0], n.stack(2, 2)[:, 1]
     check('backward', (got - u * g[:, 1]) / (u * total[:, 1]), most=narrow + 1.0)
     n.close()
 

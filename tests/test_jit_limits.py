@@ -13,6 +13,7 @@ from cpde_amd import hip, workloads as W
     (3, 5, [3, 208, 208, 8], 8192),        # 56 rows: one point
     (3, 5, [3, 208, 208, 1], 8192),        # and two, just below 160 KB
     (2, 6, [2, 80, 256, 1], 8192),         # 28 rows, two points
+    (2, 6, [2, 128, 240, 1], 8192),
     (2, 6, [2, 128, 256, 8], 1000),
 ])
 def test_modules_at_the_lds_limit_compile(tmp_path, monkeypatch, variables, order, neurons, width):
