@@ -44,9 +44,16 @@ PUBLISHED_POINTS_DERIVS_PER_S = 729 * 28 / 5.65e-3
 # (forward, loss, weight gradient) per derivative order (README.md:57-63).
 PUBLISHED_MS = {0: 0.41, 1: 0.68, 2: 1.10, 3: 1.72, 4: 2.40, 5: 3.59, 6: 5.65}
 PEAK_FP32_MFMA = 157.3e12   # flop/s, dense
+PEAK_SPLIT_MFMA = 2.5e15 / 6  # of products on split operands: six bf16 products each
 PEAK_HBM = 8.0e12           # bytes/s
 MFMA_KINDS = {'gemm_forward', 'gemm_transposed', 'gemm_wgrad', 'fused_forward', 'fused_backward', 'network_forward',
               'network_backward', 'network_epoch'}
+# The kernel classes that multiply on split operands, per workload (the others:
+# the fp32 matrix instruction): layers of 128 and more in the network kernels,
+# weight gradients of long splits.
+NETWORK_KINDS = {'network_forward', 'network_backward', 'network_epoch'}
+SPLIT_KINDS = {**{f'fourier_fit_order{k}': NETWORK_KINDS for k in range(7)}, 'poisson_disk_order2': set(),
+               'fourier_3d_order4': NETWORK_KINDS | {'gemm_wgrad'}, 'fourier_large_order6': NETWORK_KINDS | {'gemm_wgrad'}}
 # CPU baseline sample: about this many multiply-adds of the linear steps
 # (rows x points x sum of n_in*n_out), ~12 s of the reference CPU server on
 # one core of the benchmark host.
@@ -120,6 +127,19 @@ def traffic(workload, kind):
     return round(kib[0] * 1024 * COPY_SCALE[0] + kib[1] * 1024 * COPY_SCALE[1])
 
 
+def mfma_peak(workload, kind):
+    return PEAK_SPLIT_MFMA if kind in SPLIT_KINDS[workload] else PEAK_FP32_MFMA
+
+
+def epoch_roof(wl, workload):
+    """Seconds of an epoch's linear steps at the peaks of the instructions that
+    they run on (weight gradients: as many operations as the forward), and of its
+    bytes."""
+    wgrad = 2.0 * linear_macs(wl)
+    return (wgrad / mfma_peak(workload, 'gemm_wgrad') +
+            (wl.flops_per_epoch() - wgrad) / mfma_peak(workload, 'network_epoch') + wl.bytes_per_epoch() / PEAK_HBM)
+
+
 def roofline(report, workload):
     """Dominant kernel class by device time; achieved = its algorithmic work
     per launch divided by its mean launch duration; traffic = its measured HBM
@@ -128,7 +148,7 @@ def roofline(report, workload):
     launches, ms, work = report[kind]
     seconds = ms / 1e3
     if kind in MFMA_KINDS:
-        achieved, peak, unit, bound = work / seconds / 1e12, PEAK_FP32_MFMA / 1e12, 'TFLOP/s', 'mfma'
+        achieved, peak, unit, bound = work / seconds / 1e12, mfma_peak(workload, kind) / 1e12, 'TFLOP/s', 'mfma'
     else:
         achieved, peak, unit, bound = work / seconds / 1e9, PEAK_HBM / 1e9, 'GB/s', 'hbm'
     return {'kernel': kind, 'bound': bound, 'achieved': round(achieved, 3), 'peak': peak, 'unit': unit,
@@ -337,7 +357,7 @@ def other_workloads(names, settle_ms):
         wl = spec.make()
         run = run_server if spec.server else run_direct
         ms, device_ms, _, _, report, settled = run(wl, spec.steps, spec.warmup, spec.trace_steps, settle_ms)
-        t_roof = wl.flops_per_epoch() / PEAK_FP32_MFMA + wl.bytes_per_epoch() / PEAK_HBM
+        t_roof = epoch_roof(wl, name)
         out[name] = {'config': describe(wl, name), 'steps': spec.steps, 'warmup': spec.warmup,
                      'ms_per_step': round(ms, 4),
                      'device_ms_per_step': None if device_ms is None else round(device_ms, 4),
@@ -385,7 +405,7 @@ def main(argv=None):
     ms, device_ms, loss, device, report, settled = runner(wl, steps, warmup, trace_steps, args.settle_ms)
 
     value = point_rows(wl) / (ms / 1e3)
-    t_roof = wl.flops_per_epoch() / PEAK_FP32_MFMA + wl.bytes_per_epoch() / PEAK_HBM
+    t_roof = epoch_roof(wl, args.workload)
     out = {
         'metric': METRIC,
         'value': round(value, 1),

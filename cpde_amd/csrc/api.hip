@@ -337,9 +337,9 @@ static bool one_pass_any_length(const std::vector<int>& neurons) {
 // tile is written over its operand tile, so a workgroup needs no more LDS
 // than one point did.  That needs whole columns per composition lane (hidden
 // widths above 64) and hidden widths that are multiples of 16.  Measured:
-// 3->128^5->1 over 32,768 points 6.87 -> 5.79 ms per epoch, 2->256^4->1 over
-// 65,536-point chunks 102.8 -> 95.4 ms; 2->128^4->1 at 729 points (under one
-// workgroup per CU either way): two points per workgroup were slower.
+// 3->128^5->1 over 32,768 points 5.06 -> 4.43 ms per epoch, 2->256^4->1 over
+// 65,536 19.5 -> 16.8, 2->128^4->1 at order 6 over 8,192 0.824 -> 0.777; over 729
+// (729 workgroups, or 365) two points per workgroup were slower, 0.072 -> 0.119.
 static FusedTuning tuning(int rows, int width, int compute_units, const std::vector<int>& neurons) {
     FusedTuning t;
     int npb = rows <= 16 ? 32 / rows : 1;
@@ -355,7 +355,8 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
             pair.col_tile = 16;
             pair.max_split = 1;  // one tile needs whole columns per lane, of a layer beside a wider one too
             // Split products of layers wider than 128 leave room for one workgroup
-            // per CU: eight waves (2->256^4->1, order 6: 74.5 -> 68.1 ms per epoch).
+            // per CU: eight waves (2->256^4->1 at order 6 over 65,536 points 18.4 ->
+            // 16.8 ms per epoch; 3->128^5->1 over 32,768 stays at four, 4.43 -> 5.58).
             if (split_products(neurons) && *std::max_element(neurons.begin() + 1, neurons.end() - 1) > 128)
                 pair.net_threads = 512;
             // Split operands are half as large again as fp32 ones: 56 rows of
@@ -382,19 +383,19 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // workgroup runs eight waves per workgroup: with one wave per SIMD the
     // matrix-core and load latencies of the layer chain have nothing to hide
     // behind.  2->128^4->1 over 729 points (three points per workgroup, 243
-    // workgroups), ms per epoch at orders 0..3: 0.0416 -> 0.0409, 0.0454 ->
-    // 0.0445, 0.0500 -> 0.0487, 0.0576 -> 0.0563.  With more workgroups than
-    // CUs it was slower (order 4, 365 workgroups: 0.0700 -> 0.0742).
+    // workgroups), us per epoch at orders 0..3: 29.5 -> 28.0, 35.8 -> 33.0, 45.3 ->
+    // 41.5, 52.0 -> 47.3; on fp32 products, 2->128->64->128->1, 22.6 -> 22.4, 24.4 ->
+    // 24.3, 29.4 -> 29.1, 33.6 -> 32.7.  With more workgroups than CUs it was
+    // slower (2->128^4->1 at order 4, 365 workgroups: 56.2 -> 58.5).
     if (width > 0 && rows <= 16 && npb > 1 && !value_leaf && (width + npb - 1) / npb <= compute_units)
         t.net_threads = 512;
     t.net_threads = env_int("CPDE_NET_THREADS", t.net_threads) == 512 ? 512 : 256;
     // The waves of a workgroup share a layer's fp32 products by output tile.  Where
     // 32x32 tiles of the narrowest hidden layer are fewer than the waves (a
     // 128-wide layer in eight waves, a 64-wide one in four), 16-column tiles
-    // keep every wave busy.  2->128^4->1 over 729 points, ms per epoch with
-    // 32 -> 16 columns: order 0 (eight waves) 0.0412 -> 0.0353, order 1
-    // 0.0448 -> 0.0384, order 2 0.0491 -> 0.0467, order 3 0.0567 -> 0.0525;
-    // order 4 (four waves, four tiles) 0.0700 -> 0.0719, so 32 stays there.
+    // keep every wave busy.  2->128->64->128->1 over 729 points, us per epoch with
+    // 32 -> 16 columns at orders 0..4: 25.5 -> 22.4, 27.5 -> 24.3, 30.6 -> 29.1,
+    // 35.2 -> 32.7, 42.8 -> 39.0.
     // Columns that fit in 16 take 16 in any case: a 32-column tile would be
     // half padding.
     if (t.col_tile == 0 && t.net_points_per_block > 1 && neurons.size() >= 3) {
@@ -407,9 +408,9 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     // Whole compositions per lane, except for several-point workgroups of up
     // to 32 rows, where a split over lanes fills the waves: on the Taylor-scaled
     // rows of one point per workgroup the split only adds lanes that repeat the
-    // jet (2->128^4->1 over 729 points, ms per epoch with a split of two against
-    // none: order 5 (21 rows) 0.0936 / 0.0904, order 6 (28 rows) 0.1036 /
-    // 0.0992; orders 1-4, several points per workgroup, within 0.3 %).
+    // jet (2->128^4->1 over 729 points, us per epoch with a split of two against
+    // none: order 5 (21 rows) 64.3 / 63.0, order 6 (28 rows) 75.1 / 72.4; orders
+    // 0-4, several points per workgroup, within 0.3 %).
     const bool whole = rows > 32 || (rows > 16 && t.net_points_per_block == 1);
     // (Where whole compositions leave three lanes of four idle, and CUs without a
     // second workgroup, the mirror split still pays: 2->32^2->1 at order 6 over 40
@@ -425,9 +426,9 @@ static FusedTuning tuning(int rows, int width, int compute_units, const std::vec
     t.col_tile = env_int("CPDE_NET_COLTILE", t.col_tile);
     // Paired neuron blocks in the 16-column products (weight operands as
     // float2, one LDS operand read per two products), on wherever a layer's
-    // width is a multiple of 32 per wave.  Measured, ms per epoch against the
-    // single blocks: 2->128^4->1 order 6 at 729 points 0.0952 / 0.0963, order 5
-    // 0.0879 / 0.0876, 3->128^5->1 order 4 at 32768 points 5.20 / 5.37.
+    // width is a multiple of 32 per wave.  Measured, us per epoch against the
+    // single blocks, order 6 at 729 points: 2->128->256->128->1 134.7 / 137.5,
+    // 2->128^2->64->1 55.5 / 57.4; order 5, 2->128->64->128->1 43.1 / 43.5.
     t.b_pairs = env_int("CPDE_NET_BPAIR", t.b_pairs);
     t.scaled = env_int("CPDE_SCALED", t.scaled) ? 1 : 0;
     // Wave priorities by dispatch round (tier_raise in the generated source).

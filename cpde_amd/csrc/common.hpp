@@ -485,7 +485,8 @@ inline size_t weight_operands(int n_in, int n_out) {
 // The operands of `count` weight blocks in one launch (their padding is left alone).
 void launch_weight_operands(Device& d, const float* const* W, void* const* WS, const int* n_in, const int* n_out,
                             int count, bool split);
-// Fixed-order sum of `blocks` per-workgroup cost records into cost slot cost_index.
+// More than kMaxCostBlocks per-workgroup cost records, in order, into at most that
+// many at `out`, which one workgroup finishes (ReduceArgs); returns their number.
 int launch_stage_cost(Device& d, const CostStats* partials, int blocks, CostStats* out);
 // Zero the slots among [0, count) still marked fresh (before something reads them on the device).
 void launch_clear_fresh(Device& d, int count);

@@ -528,16 +528,17 @@ __device__ __forceinline__ int xcd_item(const WgradArgs& a, int t) {
 // An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 significant
 // bits): x = x1 + x2 + x3, x1 its upper half, x2 the rest rounded to nearest,
 // x3 what remains.  Of the nine products of two such sums, six matter at 24
-// bits: x1 y1 goes into one accumulator and x1 y2 + x2 y1 + x2 y2 + x1 y3 +
-// x3 y1 into another, so that the small terms are not rounded to the large
-// sum's last place; the two meet once at the end.  v_mfma_f32_16x16x32_bf16
+// bits: x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1, then x1 y1.  Every step of 32
+// columns sums its six, the small ones first, from zero (split_products), so that
+// they are not rounded to the running sum's last place, and adds that once to the
+// running sum.  v_mfma_f32_16x16x32_bf16
 // runs at 2,100 TFLOP/s here and v_mfma_f32_16x16x4_f32 at 153, so six of
 // them cost 0.44 of one fp32 product, and bf16 products overlap with other
 // waves' vector instructions, which fp32 ones do not (0.26 + 0.91 ms alone,
-// 1.00 together; fp32 0.22 + 0.91, 1.13).  Relative error of a product
-// against 64 bits: 128 random terms 6.0e-8 (fp32 instruction 1.9e-7), 28,672
-// terms of one sign 8.6e-7 (2.4e-6; 7.1e-6 with one accumulator for all six).
-// An infinite operand gives NaN where fp32 gave an infinity (inf - inf).
+// 1.00 together; fp32 0.22 + 0.91, 1.13).  Error against 64 bits, rms in units of
+// 2^-24 of the terms' norm: products of 261 and 300 terms 1.0 (fp32 instruction 3.5
+// to 3.9), weight gradients of 36,000 columns 3.9 and 4.1 (3.8 and 6.6).  An
+// infinite operand gives NaN where fp32 gave an infinity (inf - inf).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
