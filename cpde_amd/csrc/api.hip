@@ -811,17 +811,21 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
     // weight gradient per epoch (19.1 with 128x128 tiles, two per CU); 2->512^3->1 over
     // 12,288 columns 160 -> 125 us.  They need the tile filled, by as many direct tiles
     // as cost more: ten, eight where a width off 64 masks those (at order 6 over 8,192
-    // points, direct and split: 128->256 144 and 170 us, 384->384 652 and 733, 300->300
-    // 627 and 716; 512->300 1,053 and 758, 256->70 255 and 184, 200->200 333 and 180),
-    // and 256 columns a split, as a split's partials are 16 direct tiles' (512->512
-    // over 4,374 columns, 68 a split, 47 and 58 us; over 12,288, 192, 89 and 82;
-    // 384->384 over 12,288 59 and 72).
+    // points, direct and split: 128->256 144 and 170 us, 192->192 171 and 183, 300->300
+    // 627 and 716; 256->256 266 and 202, 256->70 255 and 184, 200->200 333 and 180), and
+    // 256 columns a split, as a split's partials are 16 direct tiles' (256->256 over
+    // 300 columns 18 and 29 us, 130->130 over 4,374 21 and 29, 256->256 over 120,000, 469
+    // a split, 167 and 130).
     //   128x128 tiles otherwise, at 512 columns a split: 3->128^5->1 over 32,768
     // points 1.32 -> 0.98 ms, the stacks' bytes at the rate of a copy; with 240
     // (2->128^4->1, 20,412 columns) the direct tiles stay ahead, 22 against 27 us.
     // Beside direct tiles in the launch one takes 2.5 times as long over a column,
     // and as many more splits, and pays for masked widths alone (2->96^2->64->1 at order
     // 6 over 8,192 points 167 -> 139 us, 2->128->64->128^2->1 174 -> 191).
+    //   Plans outside the network-fused kernels keep split tiles where they are slower
+    // too (300->300 above): their sums are a third as far from 64 bits as the direct
+    // tiles' (1->438^2->1 at order 2 over 3,314 points 5.4e-8 and 1.5e-7).
+    const bool layers = !p.fused;
     auto cost = [&](int t) { return staged || t == 64 ? 2 : t == 128 ? 5 : 0; };  // in the launch of the smaller tiles
     auto exact = [&](int k) { return widths(k).first % 64 == 0 && widths(k).second % 64 == 0; };
     auto clear_split = [&](int size) {
@@ -832,13 +836,14 @@ static GradientPlan plan_gradients(Plan& p, bool accumulate, const int* external
         for (int k = 0; k < T; ++k) {
             if (!tile[k] || widths(k).first <= 64) continue;
             if (widths(k).second <= 128) tile[k] = 128;
-            else if (tiles_at(k, 64) >= (exact(k) ? 10 : 8) * tiles_at(k, 256)) tile[k] = 256;
+            else if (layers || tiles_at(k, 64) >= (exact(k) ? 10 : 8) * tiles_at(k, 256)) tile[k] = 256;
         }
-        if (double(K) * count_tiles([](int t) { return t == 256; }) < 256.0 * d.compute_units) clear_split(256);
-        if (std::count(tile.begin(), tile.end(), 64))
+        const double columns256 = double(K) * count_tiles([](int t) { return t == 256; });
+        if (!layers && columns256 < 256.0 * d.compute_units) clear_split(256);
+        if (!layers && std::count(tile.begin(), tile.end(), 64))
             for (int k = 0; k < T; ++k)
                 if (tile[k] == 128 && exact(k)) tile[k] = 64;
-        if (double(K) * count_tiles(cost) < 512.0 * 5 * d.compute_units) clear_split(128);
+        if (!(layers && columns256 > 0) && double(K) * count_tiles(cost) < 512.0 * 5 * d.compute_units) clear_split(128);
     }
     auto has = [&](int size) { return !staged && std::count(tile.begin(), tile.end(), size) > 0; };
     // whole waves of tiles: a partial last wave would run alone for a whole split

@@ -18,8 +18,9 @@ pytestmark = pytest.mark.gpu
     (1, [2, 96, 96, 64, 1], 60013),        # masked 128 tiles beside direct ones
     (1, [2, 128, 128, 64, 1], 60013),      # whole ones: direct all
     (1, [2, 256, 70, 66, 1], 60013),       # 256 and 128 tiles
-    (0, [2, 512, 512, 264, 1], 20001),     # 256 tiles where they are filled
-    (0, [2, 512, 512, 1], 700),            # too few columns for them
+    (1, [2, 130, 130, 1], 700),            # too few columns for a 256 tile
+    (0, [2, 512, 512, 264, 1], 20001),     # outside the network kernels: 256 tiles all the same
+    (0, [2, 512, 512, 1], 700),
 ])
 def test_mixed_widths(device, order, neurons, points):
     wl = workload(2, order, neurons, points, 0, seed=73)
