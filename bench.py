@@ -60,22 +60,22 @@ SPLIT_KINDS = {**{f'fourier_fit_order{k}': NETWORK_KINDS for k in range(7)}, 'po
 CPU_SAMPLE_MACS = 3.0e9
 
 # HBM bytes per launch from rocprofv3 counter passes over this benchmark
-# (profiles/network_kernels_traffic.md; poisson_disk_order2: _counters.md): mean FETCH_SIZE and
+# (profiles/network_kernels_traffic.md): mean FETCH_SIZE and
 # WRITE_SIZE in KiB per dispatch, scaled by what the same counters read for a
 # plain 256 MiB copy (``--copy-calibration``): 268,435,456 B / 131,084.475 KiB
 # read, 268,435,456 B / 262,144 KiB written.
 COPY_SCALE = (268435456 / (131084.475 * 1024), 268435456 / (262144 * 1024))
 TRAFFIC_KIB = {
-    'fourier_fit_order2': {'network_epoch': (5843.1, 25788.75), 'gemm_wgrad': (7327.5, 3954.0),
-                           'split_reduce': (3974.35, 4377.12)},
-    'fourier_fit_order6': {'network_epoch': (18758.46, 113939.95), 'gemm_wgrad': (34724.46, 4147.5),
-                           'split_reduce': (4561.9, 4377.12)},
-    'poisson_disk_order2': {'network_epoch': (6934.3, 54427.2), 'gemm_wgrad': (7005.0, 2946.7),
-                            'split_reduce': (1940.5, 261.7)},
-    'fourier_3d_order4': {'network_forward': (102824.02, 5739264.75), 'network_backward': (1827527.51, 3215728.27),
-                          'gemm_wgrad': (2326641.64, 33273.6), 'split_reduce': (37114.11, 1120.4)},
-    'fourier_large_order6': {'network_backward': (5195012.63, 8391610.28), 'network_forward': (602051.27, 14687232.0),
-                             'gemm_wgrad': (5603621.21, 66699.63)},
+    'fourier_fit_order2': {'network_epoch': (5842.6, 25788.75), 'gemm_wgrad': (7329.5, 3954.0),
+                           'split_reduce': (3974.78, 4377.12)},
+    'fourier_fit_order6': {'network_epoch': (18889.32, 113941.78), 'gemm_wgrad': (34718.48, 4147.5),
+                           'split_reduce': (4562.51, 4377.12)},
+    'poisson_disk_order2': {'network_epoch': (5851.24, 42232.76), 'gemm_wgrad': (10013.67, 4228.28),
+                            'split_reduce': (2625.05, 261.71)},
+    'fourier_3d_order4': {'network_forward': (103959.18, 5739265.41), 'network_backward': (1827880.57, 3224208.74),
+                          'gemm_wgrad': (2326643.74, 33276.07), 'split_reduce': (37110.12, 1117.04)},
+    'fourier_large_order6': {'network_backward': (5195014.02, 8391673.16), 'network_forward': (601986.04, 14687232.0),
+                             'gemm_wgrad': (5603621.32, 66650.4)},
 }
 
 
