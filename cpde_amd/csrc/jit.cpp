@@ -852,10 +852,14 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
     // the last hidden layer's y (read from X by the output layer's partial) and
     // the first one's dE/dz (read from X by the input transition's) stay in the
     // workgroup: no later launch reads them
-    const std::string unread = tuning.keep_asked ? ", kAsked" : ", kDropped";
+    auto asked = [&](int layer, const char* stacks) {
+        if (tuning.keep_asked)
+            ep << "    net_keep_stack<" << neurons[layer] << ">(a, a." << stacks << "[" << layer << "], X, p0, npts);\n";
+    };
     for (int t = 1; t + 2 < L; ++t)
         ep << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
-           << (t + 3 == L ? unread : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+           << (t + 3 == L ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+    if (L > 3) asked(L - 2, "Y");
     const std::string last = std::to_string(neurons[L - 2]);
     ep << "    UAhead<" << last << ", output_adjoint_split<" << last
        << ">()> ua;  // the last hidden layer's u rows, in flight during the output layer and the cost\n"
@@ -869,7 +873,8 @@ static std::string epoch_body(const std::vector<int>& neurons, const std::string
        << "    tier_drop();\n";
     for (int t = L - 3; t >= 1; --t)
         ep << "    net_hidden_backward<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t > 1)
-           << (t == 1 ? unread : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+           << (t == 1 ? ", false" : "") << ">(a, " << t << ", X, T, p0, npts);\n";
+    if (L > 3) asked(1, "G");
     ep << "    net_input_gradient<" << neurons[0] << ", " << neurons[1] << ", true>(a, X, p0, npts, xin);\n";
     // Diagnostics (FusedTuning::stamps): a clock stamp after every phase --
     // each call above and each barrier between them -- written over the
@@ -922,7 +927,7 @@ std::string fused_source(const Tables& t, const std::vector<int>& neurons, const
         << "    __syncthreads();\n";
     for (int t = 1; t + 2 < L; ++t)
         val << "    net_hidden<" << neurons[t] << ", " << neurons[t + 1] << ", " << operand(t + 3 < L)
-            << ", kDropped, false>(a, " << t << ", X, T, p0, npts);\n";
+            << ", false, false>(a, " << t << ", X, T, p0, npts);\n";
     val << "    net_output<" << neurons[L - 2] << ", " << neurons[L - 1] << ">(a, " << L - 2 << ", X, p0, npts);\n";
     val << "    if (a.keep) {\n";
     for (int t = 0, offset = 0; t + 2 < L; ++t) {
