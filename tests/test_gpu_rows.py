@@ -1,6 +1,7 @@
 """Plans outside the fused kernels (more than 64 rows, layers wider than 256):
 the epoch of the generated row kernels and their products against the oracle,
-and against the table-driven compositions on the same plan."""
+and against the table-driven compositions on the same plan (the products'
+precision is pinned by test_gpu_product_accuracy.py)."""
 import numpy as np
 import pytest
 
