@@ -1652,6 +1652,7 @@ int cpde_net_read(cpde_net* net, int transition, int buffer, float* values) {
         flush_reduce(d);
         require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
         require(values != nullptr, "null argument");
+        if (d.capturing) sync_stream(d, __LINE__);  // refused, before anything of it is recorded
         HIP_CHECK(hipMemcpyAsync(values, net->state[buffer][transition], net->param_count(transition) * sizeof(float),
                                  hipMemcpyDeviceToHost, d.stream));
         sync_stream(d, __LINE__);
@@ -1664,6 +1665,7 @@ int cpde_net_write(cpde_net* net, int transition, int buffer, const float* value
         flush_reduce(d);
         require(transition >= 0 && transition < net->layers - 1 && buffer >= 0 && buffer < 4, "invalid state buffer");
         require(values != nullptr, "null argument");
+        if (d.capturing) sync_stream(d, __LINE__);  // refused, before anything of it is recorded
         if (buffer == 0) {
             keep_weights(*net);
             net->ws_current = false;

@@ -279,18 +279,19 @@ class Net:
         check(load().cpde_net_state(self.handle, t, b, ctypes.byref(p), ctypes.byref(c)))
         return p, c.value
 
-    def _count(self, t):
-        assert 0 <= t < len(self.neurons) - 1
+    def _count(self, t, b):
+        if not 0 <= t < len(self.neurons) - 1:
+            self.state_ptr(t, b)   # the library's refusal
         return self.neurons[t + 1] * (self.neurons[t] + 1)
 
     def state(self, t, b):
-        v = np.empty(self._count(t), np.float32)
+        v = np.empty(self._count(t, b), np.float32)
         check(load().cpde_net_read(self.handle, t, b, _ptr(v)))
         return v
 
     def set_state(self, t, b, values):
         v = np.ascontiguousarray(values, np.float32)
-        assert v.size == self._count(t)
+        assert v.size == self._count(t, b)
         check(load().cpde_net_write(self.handle, t, b, _ptr(v)))
 
     def active(self, t):

@@ -55,13 +55,24 @@ def test_operands_are_rebuilt_after_a_write_alone(device):
     f.net.set_state(1, 0, f.wl.init[1])
     f.run()
     assert np.array_equal(f.outputs(), first)
-    f.close()
+    # refused while a capture is open, which records nothing of it
+    device.capture_begin()
+    for refused in (lambda: f.net.state(1, 0), lambda: f.net.set_state(1, 0, np.zeros_like(f.wl.init[1]))):
+        with pytest.raises(hip.CpdeError) as e:
+            refused()
+        assert e.value.code == hip.EINVAL
+    f.run()
+    replay = device.capture_end()
+    replay.launch()
+    assert np.array_equal(f.outputs(), first)
+    replay.destroy()
     for bad in ((3, 0), (0, 4), (-1, 0)):
-        f = hip.Net(device, [2, 8, 8, 1], [1, 0, 0, 1])
         v = np.zeros(1024, np.float32)
         for call in (hip.load().cpde_net_read, hip.load().cpde_net_write):
-            assert call(f.handle, *bad, v.ctypes.data) == hip.EINVAL
-        f.destroy()
+            assert call(f.net.handle, *bad, v.ctypes.data) == hip.EINVAL
+        with pytest.raises(hip.CpdeError):
+            f.net.state(*bad)
+    f.close()
 
 
 @pytest.mark.parametrize('width', [128, 40])
