@@ -2205,8 +2205,10 @@ int cpde_update_resolve(cpde_device* dev, cpde_cost_stats* cost_out, cpde_gradie
                                 u.graph ? dev->host_graph_summary : nullptr};
         *updated = update_accepted(guard) ? 1 : 0;
         if (!*updated) {  // the update did not apply: RPROP's buffers switch back
+            // (operands rewritten in between, for other weights, are not current either)
+            const bool current = u.net->ws_current && u.ws_current;
             if (u.rprop) rprop_done(*u.net);
-            u.net->ws_current = u.ws_current;
+            u.net->ws_current = current;
         }
     });
 }

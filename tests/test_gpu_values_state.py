@@ -234,3 +234,29 @@ def test_backward_of_another_plan_reads_the_arena(device):
         other.close()
         v.close()
     same(*got)
+
+
+def test_operands_after_a_rejected_update(device):
+    """Stacks of an older forward asked for between an update's issue and its
+    rejection: the next forward runs on the weights that stand."""
+    neurons = [2, 128, 130, 1]
+    v = Values(device, neurons)
+    T = len(neurons) - 1
+    v.forward(0.25)
+    for t, w in enumerate(v.wl.init):
+        v.net.set_state(t, 0, 0.5 * w)
+    kept = hip.vp()
+    hip.check(hip.load().cpde_stacks_create(v.plan.handle, hip.ctypes.byref(kept)))
+    hip.check(hip.load().cpde_plan_bind(v.plan.handle, kept))
+    want = v.forward(0.25).output()   # the operands are current
+    hip.check(hip.load().cpde_plan_bind(v.plan.handle, None))
+    for t in range(T):
+        v.net.set_state(t, v.net.active(t), np.full_like(v.wl.init[t], np.inf))
+    device.costs_begin(1)
+    v.net.issue_update(1, inspect='full')
+    v.plan.stack_ptr(1, 1)
+    assert not v.net.resolve_update(1)[2]
+    v.plan.forward()
+    same([v.output()], [want])
+    hip.check(hip.load().cpde_stacks_destroy(kept))
+    v.close()
